@@ -1,0 +1,32 @@
+// FP64 matrix-core products of the density-fitted exchange (mjk_dfgemm.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+namespace mjk {
+
+// Split of a long-inner-dimension product C = A^T B (C n x n, A and B k-major
+// columns of length kin): 64 x 64 tiles x nsplit slices of the inner dimension.
+struct TnPlan {
+    int nt = 0;            // tiles per dimension
+    int ntile = 0;         // tiles computed (the lower triangle when C is symmetric)
+    int nsplit = 0;        // slices of the inner dimension, a multiple of 8 (one XCD each)
+    long long kc = 0;      // inner length of a slice, a multiple of 16
+    size_t ws = 0;         // workspace doubles
+};
+TnPlan df_tn_plan(int n, long long kin, bool sym);
+
+// C (n x n, column-major) = A^T B; sym: A == B, the lower tiles computed and
+// mirrored.  part: plan.ws doubles.
+int df_tn(const TnPlan& plan, const double* A, const double* B, int n, long long kin, bool sym, double* part,
+          double* C, hipStream_t st);
+
+// Y_i (naux x ncol, column-major) = B_i X for i < nao, B_i the naux x nao
+// column-major block at B + i naux nao; X given transposed and padded by df_pad_x.
+int df_y(const double* B, const double* Xp, int nao, int naux, int ncol, double* Y, hipStream_t st);
+
+// doubles of the padded copy of X, and the copy: X(l, o) at src[l sl + o so]
+size_t df_xp_size(int nao, int ncol);
+int df_pad_x(const double* src, long long sl, long long so, int nao, int ncol, double* Xp, hipStream_t st);
+
+}  // namespace mjk

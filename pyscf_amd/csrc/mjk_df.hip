@@ -13,11 +13,12 @@
 // Builds (per call):
 //   * J: rho = B vec(D) and vec(J) = B^T rho, two bandwidth-bound passes over
 //     the lower-triangle rows of B (k_df_rho, k_df_j);
-//   * K of a density: Y_i = B_i D^T for every i (one strided-batched GEMM,
-//     B_i = the naux x nao block of row i), then K = B^T Y as one GEMM over
-//     (P, l): K_ik = sum_Pl B_k[P,l] Y_i[P,l] = sum_P (B_P D B_P)_ik;
+//   * K of a density: Y_i = B_i D^T for every i (B_i = the naux x nao block of
+//     row i), then K = B^T Y over (P, l): K_ik = sum_Pl B_k[P,l] Y_i[P,l] =
+//     sum_P (B_P D B_P)_ik;
 //   * K of occupied orbitals X (D = X X^T): Y_i = B_i X, K = Y^T Y.
-// All on rocBLAS/rocSOLVER on the context's stream; FP64 throughout.
+// Both K products on the FP64 matrix cores (mjk_dfgemm.hip); the fit on
+// rocBLAS/rocSOLVER; everything on the context's stream, FP64 throughout.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
@@ -29,6 +30,7 @@
 #include <vector>
 
 #include "df_device.h"
+#include "df_gemm.h"
 #include "mjk.h"
 #include "mjk_internal.h"
 #include "units.h"
@@ -51,9 +53,10 @@ struct mjk_df {
     size_t caprho = 0;
     void* ws = nullptr;
     size_t capws = 0;
-    // blocks of the exchange product from the occupied orbitals (0: by size;
-    // MJK_DF_KBLOCKS overrides)
-    int kblocks = 0;
+    double* X = nullptr;       // padded orbitals (or density) of the half transform
+    size_t capX = 0;
+    double* part = nullptr;    // slices of the exchange product
+    size_t cappart = 0;
 };
 
 namespace {
@@ -103,11 +106,14 @@ __global__ void k_df_auxsph(const double* __restrict__ S, long long lds, double*
 // one column they ran at a few percent of HBM bandwidth.
 //   rho[P] = sum_{i>=j} w_ij B[ij][P],  w_ij = D_ij + D_ji (i > j), D_ii (i = j)
 // Grid: x = chunks of DF_ROWS lower-triangle rows, y = column tiles of
-// DF_COLS columns; a lane keeps DF_COLS / 256 column sums over the chunk's
-// rows, then adds them into rho (FP64 atomics; rho is zeroed first).
+// DF_COLS columns.  The chunk's weights and row positions are put in LDS once;
+// a lane keeps two neighbouring column sums over the chunk's rows, then adds
+// them into rho (FP64 atomics; rho is zeroed first).  Bandwidth-bound: tiles
+// of 512 columns leave little of the last one empty and give several blocks
+// per CU.
 constexpr int DF_ROWS = 256;
-constexpr int DF_CPT = 8;                 // columns per lane
-constexpr int DF_COLS = 256 * DF_CPT;     // columns per block
+constexpr int DF_COLS = 512;              // columns per block, two per lane
+typedef double df_d2 __attribute__((ext_vector_type(2), aligned(8)));
 
 __device__ __forceinline__ void tri_index(long long t, int& i, int& j)
 {
@@ -121,32 +127,32 @@ __device__ __forceinline__ void tri_index(long long t, int& i, int& j)
 __global__ void __launch_bounds__(256) k_df_rho(const double* __restrict__ B, int nao, int naux,
                                                 const double* __restrict__ D, double* __restrict__ rho)
 {
+    __shared__ double w[DF_ROWS];
+    __shared__ long long off[DF_ROWS];
     const long long ntri = (long long)nao * (nao + 1) / 2;
     const long long t0 = (long long)blockIdx.x * DF_ROWS;
-    const long long t1 = t0 + DF_ROWS < ntri ? t0 + DF_ROWS : ntri;
-    const int c0 = blockIdx.y * DF_COLS + threadIdx.x;
-    double acc[DF_CPT];
-#pragma unroll
-    for (int k = 0; k < DF_CPT; ++k) acc[k] = 0.0;
-    int i, j;
-    tri_index(t0, i, j);
-    for (long long t = t0; t < t1; ++t) {
-        const double w = i == j ? D[(long long)i * nao + i] : D[(long long)i * nao + j] + D[(long long)j * nao + i];
-        const double* row = B + ((long long)i * nao + j) * naux;
-#pragma unroll
-        for (int k = 0; k < DF_CPT; ++k) {
-            const int c = c0 + k * 256;
-            if (c < naux) acc[k] += w * row[c];
-        }
-        if (++j > i) {
-            ++i;
-            j = 0;
-        }
+    const int nr = (int)(t0 + DF_ROWS < ntri ? DF_ROWS : ntri - t0);
+    if (threadIdx.x < nr) {
+        int i, j;
+        tri_index(t0 + threadIdx.x, i, j);
+        w[threadIdx.x] = i == j ? D[(long long)i * nao + i] : D[(long long)i * nao + j] + D[(long long)j * nao + i];
+        off[threadIdx.x] = ((long long)i * nao + j) * naux;
     }
-#pragma unroll
-    for (int k = 0; k < DF_CPT; ++k) {
-        const int c = c0 + k * 256;
-        if (c < naux) atomicAdd(rho + c, acc[k]);
+    __syncthreads();
+    const int c = blockIdx.y * DF_COLS + 2 * threadIdx.x;
+    double a0 = 0.0, a1 = 0.0;
+    if (c + 1 < naux) {
+#pragma unroll 8
+        for (int t = 0; t < nr; ++t) {
+            const df_d2 v = *(const df_d2*)(B + off[t] + c);
+            a0 += w[t] * v.x;
+            a1 += w[t] * v.y;
+        }
+        atomicAdd(rho + c, a0);
+        atomicAdd(rho + c + 1, a1);
+    } else if (c < naux) {
+        for (int t = 0; t < nr; ++t) a0 += w[t] * B[off[t] + c];
+        atomicAdd(rho + c, a0);
     }
 }
 
@@ -508,102 +514,6 @@ int build(mjk_ctx* ctx, mjk_df* df, const int* atm, int natm, const int* bas, in
     return MJK_OK;
 }
 
-// rocBLAS's DGEMM for the long-inner-dimension shapes of the exchange
-// product (m, n = nao, inner dimension naux nocc or naux nao) runs at about
-// 50 TFLOP/s for even m and n and at a fraction of that for odd ones
-// (measured on MI355X, inner dimension 426646 and a 512 MiB workspace: m = n
-// = 730 in 9.1 ms, 729 and 731 in 68.7 ms; every odd m in 183..731 tried took
-// 68.4-68.8 ms, every even one 0.9-9.1 ms).  So the GEMMs below see even
-// dimensions only; an odd last AO is a matrix-vector product.
-
-// Block of an index in the lower-block layout of df_syrk: blocks of bs over
-// [0, ne), the odd last index (ne = nao - 1) a block of its own after them.
-__device__ __forceinline__ int df_blk(int x, int ne, int bs) { return x >= ne ? 1 << 30 : x / bs; }
-
-// Upper part of a symmetric nao x nao matrix (column-major view) whose lower
-// blocks (block of the row >= block of the column) are computed.
-__global__ void k_df_mirror(double* K, int nao, int ne, int bs)
-{
-    const long long n = (long long)nao * nao;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e / nao), r = (int)(e - (long long)c * nao);
-        if (df_blk(r, ne, bs) < df_blk(c, ne, bs)) K[e] = K[(long long)r * nao + c];
-    }
-}
-
-// Inside a workspace-size query rocBLAS calls only report sizes (statuses
-// other than success): failures count outside a query only.
-#define RBQ(ctx, query, x)                                                                            \
-    do {                                                                                              \
-        rocblas_status s_ = (x);                                                                      \
-        if (!(query) && s_ != rocblas_status_success)                                                 \
-            return ctx_fail(ctx, MJK_EDEVICE, "%s failed: %s", #x, rocblas_status_to_string(s_));     \
-    } while (0)
-
-// Blocks of the symmetric exchange product for nao AOs: one block (a single
-// GEMM) below 640 AOs, else about 250 AOs per block, a width at which the
-// GEMMs keep the full product's rate (49-57 TFLOP/s for 242-256 and 486-512
-// rows, 30 for 184, 15 for 122) while the lower triangle needs (1 + 1/nb) / 2
-// of its FLOPs.  C30H62 cc-pVDZ / cc-pVDZ-JKFIT (730 AOs, blocks 244, 244,
-// 242): the build from the occupied orbitals 21.1 -> 17.8 ms.  kblocks > 0
-// overrides.
-int df_kblocks(int nao, int kblocks)
-{
-    if (kblocks > 0) return kblocks;
-    return nao < 640 ? 1 : (nao + 125) / 250;
-}
-
-// K = Y^T Y (column-major nao x nao; Y: kin x nao, column-major) as the
-// lower blocks of nb x nb even-sized blocks over the even part of the AOs, the
-// odd last AO's row by DGEMV, then the mirror.
-int df_syrk(mjk_ctx* ctx, rocblas_handle h, int nb, int nao, int kin, const double* Y, double* K, hipStream_t st)
-{
-    const double one = 1.0, zero = 0.0;
-    const bool query = rocblas_is_device_memory_size_query(h);
-    const int ne = nao & ~1;
-    nb = std::max(1, std::min(nb, ne / 2));
-    int bs = (ne + nb - 1) / nb;
-    bs += bs & 1;   // even blocks (the last one too: ne is even)
-    for (int i0 = 0; i0 < ne; i0 += bs) {
-        const int ni = std::min(bs, ne - i0);
-        for (int j0 = 0; j0 <= i0; j0 += bs) {
-            const int nj = std::min(bs, ne - j0);
-            RBQ(ctx, query, rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, ni, nj, kin, &one,
-                                          Y + (size_t)i0 * kin, kin, Y + (size_t)j0 * kin, kin, &zero,
-                                          K + (size_t)j0 * nao + i0, nao));
-        }
-    }
-    if (ne < nao)   // row nao - 1: K[nao-1, c] = y_{nao-1} . y_c, all c
-        RBQ(ctx, query, rocblas_dgemv(h, rocblas_operation_transpose, kin, nao, &one, Y, kin, Y + (size_t)ne * kin, 1,
-                                      &zero, K + ne, nao));
-    if (query || (bs >= ne && ne == nao)) return MJK_OK;
-    k_df_mirror<<<1024, 256, 0, st>>>(K, nao, ne, bs);
-    HC(ctx, hipGetLastError());
-    return MJK_OK;
-}
-
-// K = B^T Y (column-major nao x nao; B, Y: kin x nao, column-major), even
-// GEMM dimensions: the ne x ne block by DGEMM, an odd last AO's column and
-// row by DGEMV.
-int df_gemm_tn(mjk_ctx* ctx, rocblas_handle h, int nao, int kin, const double* B, const double* Y, double* K)
-{
-    const double one = 1.0, zero = 0.0;
-    const bool query = rocblas_is_device_memory_size_query(h);
-    const int ne = nao & ~1;
-    if (ne > 0)
-        RBQ(ctx, query, rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, ne, ne, kin, &one, B,
-                                      kin, Y, kin, &zero, K, nao));
-    if (ne < nao) {
-        // column nao - 1: K[r, nao-1] = b_r . y_{nao-1}, all r
-        RBQ(ctx, query, rocblas_dgemv(h, rocblas_operation_transpose, kin, nao, &one, B, kin, Y + (size_t)ne * kin, 1,
-                                      &zero, K + (size_t)ne * nao, 1));
-        // row nao - 1: K[nao-1, c] = b_{nao-1} . y_c, c < nao - 1
-        RBQ(ctx, query, rocblas_dgemv(h, rocblas_operation_transpose, kin, ne, &one, Y, kin, B + (size_t)ne * kin, 1,
-                                      &zero, K + ne, nao));
-    }
-    return MJK_OK;
-}
-
 // J and K of n_dm densities (device, nao x nao each, row-major), optional
 // occupied orbitals X (n_dm x nao x nocc, row-major) for K
 int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, int nocc, int with_j, int with_k,
@@ -611,31 +521,10 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
 {
     mjk_ctx* ctx = df->ctx;
     hipStream_t st = mjk_internal::ctx_stream(ctx);
-    rocblas_handle h = (rocblas_handle)mjk_internal::ctx_rocblas(ctx);
-    if (!h) return ctx_fail(ctx, MJK_EDEVICE, "rocblas_create_handle failed");
-    RB(ctx, rocblas_set_stream(h, st));
-    RB(ctx, rocblas_set_pointer_mode(h, rocblas_pointer_mode_host));
     int rc;
     const int nao = df->nao, naux = df->naux;
     const long long nn = (long long)nao * nao;
-    const double one = 1.0, zero = 0.0;
     const int ncol = d_orbo ? nocc : nao;
-    // workspace of these calls (sized by a query, once per shape)
-    {
-        size_t need = 0;
-        RB(ctx, rocblas_start_device_memory_size_query(h));
-        if (ncol > 0) {
-            (void)rocblas_dgemm_strided_batched(h, rocblas_operation_none, rocblas_operation_transpose, naux, ncol, nao,
-                                                &one, df->B, naux, (rocblas_stride)naux * nao, d_dms, ncol, 0, &zero,
-                                                df->Y, naux, (rocblas_stride)naux * ncol, nao);
-            if (d_orbo)
-                (void)df_syrk(ctx, h, df_kblocks(nao, df->kblocks), nao, naux * ncol, df->Y, d_vk, st);
-            else
-                (void)df_gemm_tn(ctx, h, nao, naux * ncol, df->B, df->Y, d_vk);
-        }
-        RB(ctx, rocblas_stop_device_memory_size_query(h, &need));
-        if ((rc = workspace(df, h, need))) return rc;
-    }
     if (with_j) {
         if ((rc = grow(ctx, &df->rho, &df->caprho, (size_t)naux * n_dm))) return rc;
         HC(ctx, hipMemsetAsync(df->rho, 0, sizeof(double) * (size_t)naux * n_dm, st));
@@ -652,29 +541,29 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
         HC(ctx, hipGetLastError());
     }
     if (with_k) {
-        if ((rc = grow(ctx, &df->Y, &df->capY, (size_t)nao * naux * std::max(ncol, 1)))) return rc;
+        const long long kin = (long long)naux * ncol;
+        const TnPlan plan = df_tn_plan(nao, std::max(kin, 1LL), d_orbo != nullptr);
+        if (ncol > 0) {
+            if ((rc = grow(ctx, &df->Y, &df->capY, (size_t)nao * kin))) return rc;
+            if ((rc = grow(ctx, &df->X, &df->capX, df_xp_size(nao, ncol)))) return rc;
+            if ((rc = grow(ctx, &df->part, &df->cappart, plan.ws))) return rc;
+        }
         for (int k = 0; k < n_dm; ++k) {
             double* K = d_vk + (size_t)k * nn;
             if (ncol == 0) {
                 HC(ctx, hipMemsetAsync(K, 0, sizeof(double) * nn, st));
                 continue;
             }
-            // Y_i (naux x ncol) = B_i (naux x nao) op(M), M = D (row-major: op T) or X (row-major nao x nocc:
-            // op T; column-major, leading dimension nao: op N)
+            // Y_i (naux x ncol) = B_i (naux x nao) M, M = D or X, row-major or (orbo_colmajor) column-major
             const double* M = d_orbo ? d_orbo + (size_t)k * nao * nocc : d_dms + (size_t)k * nn;
             const bool cm = d_orbo && orbo_colmajor;
-            RB(ctx, rocblas_dgemm_strided_batched(h, rocblas_operation_none,
-                                                  cm ? rocblas_operation_none : rocblas_operation_transpose, naux,
-                                                  ncol, nao, &one, df->B, naux, (rocblas_stride)naux * nao, M,
-                                                  cm ? nao : ncol, 0, &zero, df->Y, naux, (rocblas_stride)naux * ncol,
-                                                  nao));
-            if (d_orbo) {
-                // K = Y^T Y over (P, o), symmetric
-                if ((rc = df_syrk(ctx, h, df_kblocks(nao, df->kblocks), nao, naux * ncol, df->Y, K, st))) return rc;
-            } else {
-                // K (row-major) = B^T Y over (P, l): column-major C(k, i) = K[i][k]
-                if ((rc = df_gemm_tn(ctx, h, nao, naux * nao, df->B, df->Y, K))) return rc;
-            }
+            if (df_pad_x(M, cm ? 1 : ncol, cm ? nao : 1, nao, ncol, df->X, st) ||
+                df_y(df->B, df->X, nao, naux, ncol, df->Y, st))
+                return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: half-transform launch failed");
+            // K = Y^T Y over (P, o), symmetric; or K (row-major) = B^T Y over
+            // (P, l): column-major C(k, i) = K[i][k]
+            if (df_tn(plan, d_orbo ? df->Y : df->B, df->Y, nao, kin, d_orbo != nullptr, df->part, K, st))
+                return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: exchange product launch failed");
         }
     }
     return MJK_OK;
@@ -687,7 +576,7 @@ void release(mjk_df* df)
         (void)hipStreamSynchronize(mjk_internal::ctx_stream(df->ctx));
         if (rocblas_handle h = (rocblas_handle)mjk_internal::ctx_blas(df->ctx))
             if (df->ws) (void)rocblas_set_workspace(h, nullptr, 0);
-        void* ps[] = {df->B, df->j2c, df->Y, df->D, df->rho, df->ws};
+        void* ps[] = {df->B, df->j2c, df->Y, df->X, df->part, df->D, df->rho, df->ws};
         for (void* p : ps)
             if (p) (void)mjk_device_free(df->ctx, p);
     }
@@ -731,7 +620,6 @@ int mjk_df_build(mjk_ctx* ctx, const int* atm, int natm, const int* bas, int nba
     if (env[8] != 0.0) return ctx_fail(ctx, MJK_EUNSUPPORTED, "mjk_df_build: Coulomb operator only (omega = 0)");
     mjk_df* df = new mjk_df();
     df->ctx = ctx;
-    if (const char* kb = getenv("MJK_DF_KBLOCKS")) df->kblocks = std::max(1, std::min(16, atoi(kb)));
     const int rc = build(ctx, df, atm, natm, bas, nbas, env, aux_atm, aux_natm, aux_bas, aux_nbas, aux_env, lindep);
     if (rc) {
         release(df);

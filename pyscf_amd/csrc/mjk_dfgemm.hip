@@ -1,0 +1,346 @@
+// FP64 matrix-core (v_mfma_f64_16x16x4) products of the density-fitted
+// exchange.  MI355X runs one such instruction per SIMD in 64 cycles (78.6
+// TFLOP/s), so operands read straight from memory into registers keep up: a
+// wave's 64 x 64 tile takes 16 KB of operands per 4096 matrix-core cycles, and
+// no LDS is used.
+//
+//   k_df_tn  C = A^T B over a long inner dimension (10^5 to 10^6) and a small
+//            n x n result (30 to 1500): the 64 x 64 tiles of the result are far
+//            fewer than the card's 1024 SIMDs, so the inner dimension is split
+//            over waves too, each slice's partial tile goes to a workspace and
+//            k_df_tn_sum adds the slices (a fixed order: results do not vary).
+//   k_df_y   Y_i = B_i X for every i, B_i read once: bound by the larger of
+//            reading B and the matrix cores.
+//
+// Measured on MI355X.  C18H38 cc-pVDZ (442 AOs, 73 orbitals, 2126 fitting
+// functions): K product 25.0 -> 0.58 ms (53 TFLOP/s; rocBLAS DGEMM ran it on
+// 12 tiles of 128 x 192), half transform 1.94 -> 1.56 ms (39 TFLOP/s, 43 with
+// the padding of 73 columns to 80); the J/K call 28.8 -> 3.1 ms.  A
+// nine-heavy-atom chain, def2-SVP, general density: K product 26.9 -> 0.33 ms.
+#include "df_gemm.h"
+
+#include <algorithm>
+
+namespace mjk {
+
+namespace {
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+// two doubles at 8-byte alignment: columns of odd length start there
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// Lane (m = lane % 16, q = lane / 16) of v_mfma_f64_16x16x4 holds A[m][k = q],
+// B[k = q][m], and rows 4 v + q of column m of the result in register v.
+__device__ __forceinline__ v4d mfma(double a, double b, v4d c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Sixteen inner elements k .. k + 15 of four 16-row groups: lane (m, q) takes
+// elements k + 4q .. k + 4q + 3 of row m of each group (a whole 128-byte line
+// per row over the four q), and MFMA step s multiplies elements k + 4q + s: the
+// inner index is permuted alike in both operands.
+__device__ __forceinline__ void tn_load(const double* const (&p)[4], long long k, double (&x)[4][4])
+{
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const d2u lo = *(const d2u*)(p[g] + k), hi = *(const d2u*)(p[g] + k + 2);
+        x[g][0] = lo.x;
+        x[g][1] = lo.y;
+        x[g][2] = hi.x;
+        x[g][3] = hi.y;
+    }
+}
+
+// The last, partial sixteen of a slice: n elements from k on exist for lane
+// quarter q (elements at and beyond n count zero and are not read).
+__device__ __forceinline__ void tn_load_tail(const double* const (&p)[4], long long k, int n, double (&x)[4][4])
+{
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[g][s] = s < n ? p[g][k + s] : 0.0;
+}
+
+__device__ __forceinline__ void tn_mul(const double (&a)[4][4], const double (&b)[4][4], v4d (&acc)[4][4])
+{
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = mfma(a[i][s], b[j][s], acc[i][j]);
+}
+
+// Tile t of the list: (row tile, column tile), row >= column when sym.
+__device__ __forceinline__ void tn_tile(int t, int nt, bool sym, int& ti, int& tj)
+{
+    if (!sym) {
+        ti = t % nt;
+        tj = t / nt;
+        return;
+    }
+    int r = 0;
+    while ((r + 1) * (r + 2) / 2 <= t) ++r;
+    ti = r;
+    tj = t - r * (r + 1) / 2;
+}
+
+// One wave per (tile, slice); the tiles of one slice run on one XCD (blocks go
+// to the XCDs in turn), whose L2 then serves the slice's rows to all of them.
+__global__ void __launch_bounds__(256, 1) k_df_tn(const double* __restrict__ A, const double* __restrict__ B, int n,
+                                                 long long kin, TnPlan pl, int sym, double* __restrict__ part)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, q = lane >> 4;
+    const int idx = (blockIdx.x >> 3) * 4 + wave;
+    const int s = (idx / pl.ntile) * 8 + (blockIdx.x & 7), t = idx % pl.ntile;
+    if (s >= pl.nsplit) return;
+    const long long k0 = s * pl.kc, k1 = min(k0 + pl.kc, kin);
+    int ti, tj;
+    tn_tile(t, pl.nt, sym != 0, ti, tj);
+    const double *pa[4], *pb[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {   // rows past the last are computed on the last row and dropped
+        pa[g] = A + min(ti * 64 + 16 * g + m, n - 1) * kin + 4 * q;
+        pb[g] = B + min(tj * 64 + 16 * g + m, n - 1) * kin + 4 * q;
+    }
+    v4d acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = v4d{0, 0, 0, 0};
+    double a0[4][4], b0[4][4], a1[4][4], b1[4][4];
+    long long k = k0;
+    const long long kf = k0 + ((k1 - k0) & ~15LL);   // whole sixteens (k1 < k0: none)
+    if (k + 16 <= kf) {
+        tn_load(pa, k, a0);
+        tn_load(pb, k, b0);
+        for (; k + 48 <= kf; k += 32) {   // the next sixteen in flight behind 64 MFMAs
+            tn_load(pa, k + 16, a1);
+            tn_load(pb, k + 16, b1);
+            tn_mul(a0, b0, acc);
+            tn_load(pa, k + 32, a0);
+            tn_load(pb, k + 32, b0);
+            tn_mul(a1, b1, acc);
+        }
+        tn_mul(a0, b0, acc);
+        k += 16;
+        if (k + 16 <= kf) {
+            tn_load(pa, k, a0);
+            tn_load(pb, k, b0);
+            tn_mul(a0, b0, acc);
+            k += 16;
+        }
+    }
+    if (k < k1) {
+        const int rest = (int)min(4LL, max(0LL, k1 - k - 4 * q));
+        tn_load_tail(pa, k, rest, a0);
+        tn_load_tail(pb, k, rest, b0);
+        tn_mul(a0, b0, acc);
+    }
+    double* out = part + ((long long)s * pl.ntile + t) * 4096 + lane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) out[((i * 4 + j) * 4 + v) * 64] = acc[i][j][v];
+}
+
+// Sum of the slices into C (and its mirror when sym).
+__global__ void __launch_bounds__(256) k_df_tn_sum(const double* __restrict__ part, TnPlan pl, int n, int sym,
+                                                  double* __restrict__ C)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int t = e >> 12, r = e & 4095;
+    if (t >= pl.ntile) return;
+    const double* p = part + e;
+    const long long stride = (long long)pl.ntile * 4096;
+    double v = 0.0;
+#pragma unroll 8
+    for (int s = 0; s < pl.nsplit; ++s) v += p[s * stride];
+    int ti, tj;
+    tn_tile(t, pl.nt, sym != 0, ti, tj);
+    const int lane = r & 63, u = r >> 6;   // u = (i 4 + j) 4 + v of k_df_tn
+    const int row = ti * 64 + (u >> 4) * 16 + 4 * (u & 3) + (lane >> 4);
+    const int col = tj * 64 + ((u >> 2) & 3) * 16 + (lane & 15);
+    if (row >= n || col >= n) return;
+    C[(long long)col * n + row] = v;
+    if (sym && ti != tj) C[(long long)row * n + col] = v;
+}
+
+// Y_i = B_i X.  A wave owns 64 fitting functions x (16 NSUB) orbitals of one i;
+// lane (m, q) reads four consecutive fitting functions 4m .. 4m + 3 of inner
+// element l + q (512 contiguous bytes per element over the 16 m), which are
+// row m of the wave's four 16-row groups.  The panels of one (i, row tile) are
+// neighbouring waves, so B_i comes from memory once.
+template <int NSUB>
+__global__ void __launch_bounds__(256, 1) k_df_y(const double* __restrict__ B, const double* __restrict__ Xp, int nao,
+                                             int naux, int ncol, int ldx, int npan, double* __restrict__ Y)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, q = lane >> 4;
+    const int ntm = (naux + 63) / 64;
+    const long long item = (long long)blockIdx.x * 4 + wave;
+    const int pan = (int)(item % npan);
+    const int tm = (int)((item / npan) % ntm);
+    const long long i = item / ((long long)npan * ntm);
+    if (i >= nao) return;
+    const int p0 = tm * 64 + 4 * m;
+    const bool whole = tm * 64 + 64 <= naux;   // wave-uniform
+    const double* b = B + i * nao * naux + p0 + (long long)q * naux;
+    const double* x = Xp + (long long)q * ldx + pan * 16 * NSUB + m;
+    v4d acc[4][NSUB];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int j = 0; j < NSUB; ++j) acc[g][j] = v4d{0, 0, 0, 0};
+    constexpr int U = 4;   // groups of four inner elements per step
+    const int lw = whole ? nao & ~15 : 0;
+    auto load = [&](int l, double (&ab)[U][4], double (&xb)[U][NSUB]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int le = l + 4 * u;
+            if (l < lw) {
+                const d2u lo = *(const d2u*)(b + (long long)le * naux), hi = *(const d2u*)(b + (long long)le * naux + 2);
+                ab[u][0] = lo.x;
+                ab[u][1] = lo.y;
+                ab[u][2] = hi.x;
+                ab[u][3] = hi.y;
+            } else {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    ab[u][g] = le + q < nao && p0 + g < naux ? b[(long long)le * naux + g] : 0.0;
+            }
+#pragma unroll
+            for (int j = 0; j < NSUB; ++j) xb[u][j] = x[(long long)le * ldx + 16 * j];   // rows padded to sixteens
+        }
+    };
+    auto mul = [&](const double (&ab)[U][4], const double (&xb)[U][NSUB]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int j = 0; j < NSUB; ++j) acc[g][j] = mfma(ab[u][g], xb[u][j], acc[g][j]);
+    };
+    double a0[U][4], x0[U][NSUB], a1[U][4], x1[U][NSUB];
+    load(0, a0, x0);
+    for (int l = 0; l < nao; l += 32) {   // the next sixteen elements in flight behind the products
+        if (l + 16 < nao) load(l + 16, a1, x1);
+        mul(a0, x0);
+        if (l + 16 >= nao) break;
+        if (l + 32 < nao) load(l + 32, a0, x0);
+        mul(a1, x1);
+    }
+    // lane (m, q): orbital m of sub-panel j, fitting functions 4 (4 v + q) .. + 3
+    double* y = Y + i * naux * ncol;
+#pragma unroll
+    for (int j = 0; j < NSUB; ++j) {
+        const int o = (pan * NSUB + j) * 16 + m;
+        if (o >= ncol) continue;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int p = tm * 64 + 4 * (4 * v + q);
+            double* d = y + (long long)o * naux + p;
+            if (whole) {
+                *(d2u*)d = d2u{acc[0][j][v], acc[1][j][v]};
+                *(d2u*)(d + 2) = d2u{acc[2][j][v], acc[3][j][v]};
+            } else {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    if (p + g < naux) d[g] = acc[g][j][v];
+            }
+        }
+    }
+}
+
+// Panels of the orbitals: at most six 16-column groups per wave (192
+// accumulator registers), as few panels as that allows, equally wide.
+void y_panels(int ncol, int& nsub, int& npan)
+{
+    const int n = (ncol + 15) / 16;
+    npan = (n + 5) / 6;
+    nsub = (n + npan - 1) / npan;
+}
+
+__global__ void __launch_bounds__(256) k_df_pad_x(const double* __restrict__ src, long long sl, long long so, int nao,
+                                                 int ncol, int rows, int ldx, double* __restrict__ Xp)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= rows * ldx) return;
+    const int l = e / ldx, o = e - l * ldx;
+    Xp[e] = l < nao && o < ncol ? src[l * sl + o * so] : 0.0;
+}
+
+}  // namespace
+
+// Slices: waves in whole rounds of the card's 1024 SIMDs (a wave holds a SIMD
+// to itself), at least 256 inner elements each, the count with the fullest last
+// round within eight rounds; more slices only cost workspace traffic.
+TnPlan df_tn_plan(int n, long long kin, bool sym)
+{
+    TnPlan p;
+    p.nt = (n + 63) / 64;
+    p.ntile = sym ? p.nt * (p.nt + 1) / 2 : p.nt * p.nt;
+    const long long most = std::max(1LL, kin / 256);
+    double best = -1;
+    for (int s = 8; s <= 1024; s += 8) {
+        if (s > 8 && (s > most || (long long)s * p.ntile > 8192)) break;
+        const long long waves = (long long)s * p.ntile, rounds = (waves + 1023) / 1024;
+        const double fill = (double)waves / (double)(rounds * 1024);
+        if (fill > best + 0.02) {
+            best = fill;
+            p.nsplit = s;
+        }
+    }
+    p.kc = ((kin + p.nsplit - 1) / p.nsplit + 15) / 16 * 16;
+    p.ws = (size_t)p.nsplit * p.ntile * 4096;
+    return p;
+}
+
+int df_tn(const TnPlan& pl, const double* A, const double* B, int n, long long kin, bool sym, double* part, double* C,
+          hipStream_t st)
+{
+    const int per_xcd = pl.nsplit / 8 * pl.ntile;
+    k_df_tn<<<(unsigned)((per_xcd + 3) / 4 * 8), 256, 0, st>>>(A, B, n, kin, pl, sym, part);
+    k_df_tn_sum<<<(unsigned)(pl.ntile * 16), 256, 0, st>>>(part, pl, n, sym, C);
+    return (int)hipGetLastError();
+}
+
+size_t df_xp_size(int nao, int ncol)
+{
+    int nsub, npan;
+    y_panels(ncol, nsub, npan);
+    return (size_t)((nao + 15) / 16 * 16) * (nsub * npan * 16);
+}
+
+int df_pad_x(const double* src, long long sl, long long so, int nao, int ncol, double* Xp, hipStream_t st)
+{
+    int nsub, npan;
+    y_panels(ncol, nsub, npan);
+    const int ldx = nsub * npan * 16, rows = (nao + 15) / 16 * 16;
+    k_df_pad_x<<<(unsigned)(((size_t)rows * ldx + 255) / 256), 256, 0, st>>>(src, sl, so, nao, ncol, rows, ldx, Xp);
+    return (int)hipGetLastError();
+}
+
+int df_y(const double* B, const double* Xp, int nao, int naux, int ncol, double* Y, hipStream_t st)
+{
+    int nsub, npan;
+    y_panels(ncol, nsub, npan);
+    const int ldx = nsub * npan * 16;
+    const long long items = (long long)nao * ((naux + 63) / 64) * npan;
+    const unsigned nb = (unsigned)((items + 3) / 4);
+    switch (nsub) {
+    case 1: k_df_y<1><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    case 2: k_df_y<2><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    case 3: k_df_y<3><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    case 4: k_df_y<4><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    case 5: k_df_y<5><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    default: k_df_y<6><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    }
+    return (int)hipGetLastError();
+}
+
+}  // namespace mjk

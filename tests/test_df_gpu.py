@@ -163,3 +163,31 @@ def test_device_resident_df_rhf():
     ed = dev.kernel()
     print('chain DF-RHF host %.12f device %.12f' % (eh, ed), flush=True)
     assert host.converged and dev.converged and abs(eh - ed) < 1e-9
+
+
+@pytest.mark.parametrize('size', [1, 2, 4])
+def test_exchange_matrix_core_tiles(size):
+    """The exchange products of random orbitals (1 to 7 column groups: both
+    sides of a sixteen, of a panel of six groups and of an odd inner length)
+    and of a general density against numpy on the fitted tensor; water
+    clusters of 24, 48 and 96 AOs lie on both sides of a 64-wide tile.  Sums of up to
+    1e5 products of size ~1 / 100 in 64 bits: 1e-12 of the largest element."""
+    mol = gto.M(atom=workloads.water_cluster(size, shape=(4, 1, 1)), basis='cc-pvdz')
+    d = df.DF(mol, 'weigend').build()
+    b = d.cderi()
+    nao = b.shape[1]
+    rng = numpy.random.default_rng(size)
+    for nocc in (1, 5, 16, 17, 96, 97):
+        c = rng.standard_normal((nao, nocc)) / 10
+        dm = c @ c.T
+        vj, vk = df.get_jk(d, lib.tag_array(dm, mo_coeff=c, mo_occ=numpy.ones(nocc)), 1)
+        y = numpy.einsum('pij,jo->pio', b, c, optimize=True)
+        k0 = numpy.einsum('pio,pjo->ij', y, y, optimize=True)
+        j0 = numpy.tensordot(numpy.tensordot(b, dm, 2), b, (0, 0))
+        assert abs(vk - k0).max() <= 1e-12 * abs(k0).max(), (nao, nocc)
+        assert abs(vj - j0).max() <= 1e-12 * abs(j0).max(), (nao, nocc)
+        assert (vk == vk.T).all()
+    dm = rng.standard_normal((nao, nao)) / 10
+    vj, vk = df.get_jk(d, dm, 0)
+    k0 = numpy.einsum('pij,jk,pkl->il', b, dm, b, optimize=True)
+    assert abs(vk - k0).max() <= 1e-12 * abs(k0).max()
