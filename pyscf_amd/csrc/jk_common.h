@@ -83,9 +83,20 @@ struct JKArgs {
     int diag;               // bra and ket from the same pair class: keep q <= p
     const double* Dj;       // Cartesian J densities (D + D^T), n_j slots
     const double* Dk;       // Cartesian K densities, n_k slots
-    double* J;              // accumulators J' (n_j slots); J = J' + J'^T afterwards
-    double* K;              // accumulators K' (n_k slots)
-    long long slot;         // slot stride (elements)
+    // Accumulators J' (n_j slots of jslot elements); J = J' + J'^T afterwards.  By
+    // shell pair (jpair): component f of pair q of a pair group at first-of-group +
+    // f * (pairs of the group) + (q - first pair), so that lanes holding consecutive
+    // kets add to consecutive addresses; else in the Cartesian arena.  MI355X, FP64
+    // atomics of a wave: 23.6 G lane-adds/s to 64 scattered addresses, 163-181 G to
+    // 64 consecutive ones.
+    double* J;
+    long long jslot;
+    long long jq0, jb0;     // first element of the ket's and of the bra's pair group
+    int jpair;
+    int jqn, jqp0;          // pairs and first pair of the ket's group
+    int jbn, jbp0;          // ... of the bra's group
+    double* K;              // accumulators K' (n_k slots), Cartesian arena
+    long long slot;         // slot stride of the arenas (elements)
     int n_j;
     int n_k;
     int ncopy;              // private accumulator copies (one per XCD); the kernel picks XCC_ID % ncopy
@@ -118,6 +129,29 @@ struct JKArgs {
     const int* tcount;
     int* thead;
     int ntask;
+};
+
+// One pair group's part of the J' accumulators by shell pair.
+struct JGroup {
+    long long e0;           // first element
+    int p0, n;              // first pair, pairs
+    int la, lb, ca, cb;     // components per pair: ca cb ncart(la) ncart(lb)
+};
+
+// J' by shell pair (the sum over copies) added to an accumulator in the arena.
+struct ScatterArgs {
+    const double* J;
+    long long jtot;         // elements of a slot
+    int n_j;
+    int ncopy;
+    long long jcopy;
+    double* arena;          // n_j slots of `slot` elements
+    long long slot;
+    const JGroup* groups;
+    int ngroup;
+    const int *cartA, *cartB, *pmol;
+    const long long* dbase;
+    const int* ld;
 };
 
 struct QCondArgs {

@@ -121,6 +121,17 @@ __device__ __forceinline__ void atomic_add(double* p, double v)
     unsafeAtomicAdd(p, v);
 }
 
+// Element of a J' slot: component 0 of ket pair q (Cartesian offsets oc, od);
+// component f of bra pair p, by shell pair.
+__device__ __forceinline__ long long jket_at(const JKArgs& a, int q, long long base, int ld, int oc, int od)
+{
+    return a.jpair ? a.jq0 + (q - a.jqp0) : base + (long long)oc * ld + od;
+}
+__device__ __forceinline__ long long jbra_at(const JKArgs& a, int f, int p)
+{
+    return a.jb0 + (long long)f * a.jbn + (p - a.jbp0);
+}
+
 // Load of read-only data at a wave-uniform address through the scalar cache
 // (constant address space: s_load into SGPRs), which keeps block-uniform pair
 // data out of the vector registers.
@@ -453,7 +464,7 @@ __device__ __forceinline__ void quartet_slice(const JKArgs& a, const QuartetCtx&
     const int cp = xcc_copy(a.ncopy);
     for (int s = 0; s < a.n_j; ++s) {
         const double* __restrict__ D = a.Dj + s * a.slot + base;
-        double* V = a.J + cp * a.jcopy + s * a.slot + base;
+        double* V = a.J + cp * a.jcopy + s * a.jslot;
         // J'[c,d] += sum_ab v Ds[a,b]: summed over this slice's (a, b) and the 8 bra lanes
         double dab[MA][MB];
 #pragma unroll
@@ -470,7 +481,7 @@ __device__ __forceinline__ void quartet_slice(const JKArgs& a, const QuartetCtx&
 #pragma unroll
                     for (int ib2 = IB0; ib2 < IB1; ++ib2) acc = fma(GOUT(ia, ib2, ic, id), dab[ia - IA0][ib2 - IB0], acc);
                 acc = tile_sum<8>(acc);
-                if (lane < 8 && c.qvalid && acc != 0.0) atomic_add(V + (oc + ic) * ld + od + id, acc);
+                if (lane < 8 && c.qvalid && acc != 0.0) atomic_add(V + base + (oc + ic) * ld + od + id, acc);
             }
         // J'[a,b] += sum_cd v Ds[c,d]: summed over this slice's (c, d) and the 8 ket lanes
         double dcd[MC][ND];
@@ -488,7 +499,7 @@ __device__ __forceinline__ void quartet_slice(const JKArgs& a, const QuartetCtx&
 #pragma unroll
                     for (int id = 0; id < ND; ++id) acc = fma(GOUT(ia, ib2, ic, id), dcd[ic - IC0][id], acc);
                 acc = tile_sum<1>(acc);
-                if ((lane & 7) == 0 && c.pvalid && acc != 0.0) atomic_add(V + (oa + ia) * ld + ob + ib2, acc);
+                if ((lane & 7) == 0 && c.pvalid && acc != 0.0) atomic_add(V + base + (oa + ia) * ld + ob + ib2, acc);
             }
     }
 
@@ -916,7 +927,7 @@ __attribute__((amdgpu_waves_per_eu(CoopShape<LA, LB, LC, LD>::WPE))) void k_jk_c
 #define BLK(ia, ib2, ic, id) sblk[(((ia) * NB + (ib2)) * NC + (ic)) * ND + (id)]
         for (int s = 0; s < a.n_j; ++s) {
             const double* __restrict__ D = a.Dj + s * a.slot + base;
-            double* V = a.J + cp * a.jcopy + s * a.slot + base;
+            double* V = a.J + cp * a.jcopy + s * a.jslot + base;
             double* dab = sD;
             double* dcd = sD + NA * NB;
             for (int e = tid; e < NA * NB; e += NT) dab[e] = D[(oa + e / NB) * ld + ob + e % NB];
@@ -989,7 +1000,7 @@ __attribute__((amdgpu_waves_per_eu(CoopShape<LA, LB, LC, LD>::WPE))) void k_jk_c
     if (jab_lds) {
         const int cp = xcc_copy(a.ncopy);
         for (int s = 0; s < a.n_j; ++s) {
-            double* V = a.J + cp * a.jcopy + s * a.slot + base;
+            double* V = a.J + cp * a.jcopy + s * a.jslot + base;
             for (int e = tid; e < NA * NB; e += NT) {
                 const double v = sJab[s * NA * NB + e];
                 if (v != 0.0) atomic_add(V + (oa + e / NB) * ld + ob + e % NB, v);
@@ -1074,7 +1085,9 @@ __device__ __forceinline__ void row_digest(const JKArgs& a, const QuartetCtx& c,
     const int lane = threadIdx.x & 63;
     for (int s = 0; s < a.n_j; ++s) {
         const double* __restrict__ D = a.Dj + s * a.slot + base;
-        double* V = a.J + cp * a.jcopy + s * a.slot + base;
+        // J' of this lane's ket, its components jd (and ND jd or a row) apart
+        double* V = a.J + cp * a.jcopy + s * a.jslot + jket_at(a, c.q, base, ld, oc, od);
+        const long long jd = a.jpair ? a.jqn : 1, jc = a.jpair ? (long long)ND * a.jqn : ld;
         // J'[c,d] += sum_ab v Ds[a,b]  (per quartet, global)
         double dab[MA][MB];
 #pragma unroll
@@ -1092,7 +1105,7 @@ __device__ __forceinline__ void row_digest(const JKArgs& a, const QuartetCtx& c,
 #pragma unroll
                         for (int ib2 = IB0; ib2 < IB1; ++ib2)
                             acc = fma(GOUT(ia, ib2, ic, id), dab[ia - IA0][ib2 - IB0], acc);
-                    atomic_add(V + (oc + ic) * ld + od + id, acc);
+                    atomic_add(V + ic * jc + id * jd, acc);
                 }
         }
         // J'[a,b] += sum_cd v Ds[c,d]  (summed over the wave, then into LDS)
@@ -1351,7 +1364,10 @@ __device__ __forceinline__ void row_digest_gc(const JKArgs& a, const QuartetCtx&
     gd[((ci) * CB + (cj)) * NKL + (ck) * CD + (cl)][(((ia) * NB + (ib2)) * NC + (ic)) * ND + (id)]
     for (int s = 0; s < a.n_j; ++s) {
         const double* __restrict__ D = a.Dj + s * a.slot + base;
-        double* V = a.J + cp * a.jcopy + s * a.slot + base;
+        // J' of this lane's ket and the strides of (ck, cl, ic, id)
+        double* V = a.J + cp * a.jcopy + s * a.jslot + jket_at(a, c.q, base, ld, oc, od);
+        const long long jd = a.jpair ? a.jqn : 1, jc = a.jpair ? (long long)ND * a.jqn : ld,
+                        jl = a.jpair ? (long long)NC * ND * a.jqn : ND, jk = a.jpair ? CD * jl : NC * jc;
         // J'[c,d] += sum_ab v Ds[a,b]  (per quartet and ket combination, global)
         double dab[NRA][NRB];
 #pragma unroll
@@ -1377,7 +1393,7 @@ __device__ __forceinline__ void row_digest_gc(const JKArgs& a, const QuartetCtx&
 #pragma unroll
                 for (int ib2 = 0; ib2 < NB; ++ib2)
                     acc = fma(GV(ci, cj, ck, cl, ia, ib2, ic, id), dab[ci * NA + ia][cj * NB + ib2], acc);
-                atomic_add(V + (oc + ck * NC + ic) * ld + od + cl * ND + id, acc);
+                atomic_add(V + ck * jk + cl * jl + ic * jc + id * jd, acc);
             }
         }
         // J'[a,b] += sum_cd v Ds[c,d]  (summed over the wave, then into LDS)
@@ -1686,7 +1702,9 @@ __global__ __launch_bounds__(256) void k_jk_row_gc(const JKArgs a)
         if (v == 0.0) continue;
         const int s = e / (NRA * NRB);
         const int ra = (e / NRB) % NRA, rb = e % NRB;
-        atomic_add(a.J + cp * a.jcopy + s * a.slot + base + (long long)(oa + ra) * ld + ob + rb, v);
+        const int f = (((ra / G::NA) * CB + rb / G::NB) * G::NA + ra % G::NA) * G::NB + rb % G::NB;
+        atomic_add(a.J + cp * a.jcopy + s * a.jslot +
+                       (a.jpair ? jbra_at(a, f, p) : base + (long long)(oa + ra) * ld + ob + rb), v);
     }
     __syncthreads();   // the next task rewrites the LDS rows
     }

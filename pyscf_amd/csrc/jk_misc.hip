@@ -149,6 +149,56 @@ __global__ __launch_bounds__(256) void k_sph2cart(const XformArgs x, const doubl
     }
 }
 
+// Sum of an accumulator's private copies into the first one, before the output
+// transform, which then reads one copy (it reads each element up to 36 times).
+// Bandwidth-bound.
+__global__ __launch_bounds__(256) void k_sum_copies(double* __restrict__ acc, long long n, int ncopy, long long copy)
+{
+    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
+        double v = 0.0;
+        for (int c = 0; c < ncopy; ++c) v += acc[c * copy + e];
+        acc[e] = v;
+    }
+}
+
+int launch_sum_copies(double* acc, long long n, int ncopy, long long copy, hipStream_t st)
+{
+    if (n <= 0 || ncopy < 2) return 0;
+    const long long nb = std::min<long long>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_sum_copies, dim3((unsigned)nb), dim3(256), 0, st, acc, n, ncopy, copy);
+    return (int)hipGetLastError();
+}
+
+// J' by shell pair into the arena (a group's split and merged pairs share
+// elements: atomics).  Grid: x over a slot's elements, y over slots.
+__global__ __launch_bounds__(256) void k_jscatter(const ScatterArgs a)
+{
+    const int s = blockIdx.y;
+    int g = 0;
+    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < a.jtot;
+         e += (long long)gridDim.x * blockDim.x) {
+        double v = 0.0;
+        for (int c = 0; c < a.ncopy; ++c) v += a.J[c * a.jcopy + s * a.jtot + e];
+        if (v == 0.0) continue;
+        while (g + 1 < a.ngroup && a.groups[g + 1].e0 <= e) ++g;   // e ascends
+        const JGroup G = a.groups[g];
+        const int f = (int)((e - G.e0) / G.n), p = G.p0 + (int)((e - G.e0) % G.n);
+        const int na = ncart(G.la), nb = ncart(G.lb);
+        const int comb = f / (na * nb), ia = (f / nb) % na, ib = f % nb;
+        const int m = a.pmol[p];
+        const int row = a.cartA[p] + (comb / G.cb) * na + ia, col = a.cartB[p] + (comb % G.cb) * nb + ib;
+        atomic_add(a.arena + s * a.slot + a.dbase[m] + (long long)row * a.ld[m] + col, v);
+    }
+}
+
+int launch_jscatter(const ScatterArgs& a, hipStream_t st)
+{
+    if (a.jtot <= 0 || a.n_j <= 0) return 0;
+    const unsigned nb = (unsigned)std::min<long long>((a.jtot + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_jscatter, dim3(nb, (unsigned)a.n_j), dim3(256), 0, st, a);
+    return (int)hipGetLastError();
+}
+
 // vj = C^T (J' + J'^T) C; vk = C^T (K' + K'^T) C (hermi 1) or
 // C^T (K'_D + K'_{D^T}^T) C (hermi 0, 2); hermi 2 then copies minus the lower
 // triangle into the upper one (pyscf/lib/numpy_helper.py:480-525).
@@ -156,8 +206,7 @@ __global__ __launch_bounds__(256) void k_cart2sph(const XformArgs x, const doubl
                                                   const double* __restrict__ Kc, long long cslot,
                                                   int n_dm, int hermi, int with_j, int with_k,
                                                   double* __restrict__ vj, double* __restrict__ vk,
-                                                  long long sslot, int ncopy, long long jcopy,
-                                                  long long kcopy)
+                                                  long long sslot)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int jj = blockIdx.y * blockDim.y + threadIdx.y;
@@ -185,15 +234,12 @@ __global__ __launch_bounds__(256) void k_cart2sph(const XformArgs x, const doubl
                 if (w == 0.0) continue;
                 const long long e1 = cb + (long long)(c0i + a1) * ldc + c0j + a2;
                 const long long e2 = cb + (long long)(c0j + a2) * ldc + c0i + a1;
-                for (int cp = 0; cp < ncopy; ++cp) {
-                    if (with_j) tj = fma(w, Jc[cp * jcopy + s * cslot + e1] + Jc[cp * jcopy + s * cslot + e2], tj);
-                    if (with_k) {
-                        const double* Kp = Kc + cp * kcopy;
-                        if (hermi == 1)
-                            tk = fma(w, Kp[s * cslot + e1] + Kp[s * cslot + e2], tk);
-                        else
-                            tk = fma(w, Kp[(2 * s) * cslot + e1] + Kp[(2 * s + 1) * cslot + e2], tk);
-                    }
+                if (with_j) tj = fma(w, Jc[s * cslot + e1] + Jc[s * cslot + e2], tj);
+                if (with_k) {
+                    if (hermi == 1)
+                        tk = fma(w, Kc[s * cslot + e1] + Kc[s * cslot + e2], tk);
+                    else
+                        tk = fma(w, Kc[(2 * s) * cslot + e1] + Kc[(2 * s + 1) * cslot + e2], tk);
                 }
             }
         }
@@ -325,12 +371,12 @@ int launch_sph2cart(const XformArgs& x, int maxld, const double* Dsph, long long
 
 int launch_cart2sph(const XformArgs& x, int maxnao, const double* Jc, const double* Kc, long long cslot,
                     int n_dm, int hermi, int with_j, int with_k, double* vj, double* vk, long long sslot,
-                    int ncopy, long long jcopy, long long kcopy, hipStream_t st)
+                    hipStream_t st)
 {
     dim3 blk(64, 4);
     dim3 grd((unsigned)((x.nsph_tot + 63) / 64), (unsigned)((maxnao + 3) / 4));
     hipLaunchKernelGGL(k_cart2sph, grd, blk, 0, st, x, Jc, Kc, cslot, n_dm, hermi, with_j, with_k, vj, vk,
-                       sslot, ncopy, jcopy, kcopy);
+                       sslot);
     return (int)hipGetLastError();
 }
 

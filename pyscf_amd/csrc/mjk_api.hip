@@ -58,7 +58,9 @@ int launch_sph2cart(const XformArgs& x, int maxld, const double* Dsph, long long
                     hipStream_t st);
 int launch_cart2sph(const XformArgs& x, int maxnao, const double* Jc, const double* Kc, long long cslot,
                     int n_dm, int hermi, int with_j, int with_k, double* vj, double* vk, long long sslot,
-                    int ncopy, long long jcopy, long long kcopy, hipStream_t st);
+                    hipStream_t st);
+int launch_sum_copies(double* acc, long long n, int ncopy, long long copy, hipStream_t st);
+int launch_jscatter(const ScatterArgs& a, hipStream_t st);
 int launch_compact_rows(const int4* rt, int nrt, const int* pmol, const int* active, int* list, int* count,
                         hipStream_t st);
 int launch_dmcond(const DmCondArgs& x, const double* Dsph, long long sslot, int n_dm, double* out,
@@ -384,13 +386,13 @@ struct GraphKey {
     const void* dms = nullptr;
     const void* vj = nullptr;
     const void* vk = nullptr;
-    const void* bufs[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+    const void* bufs[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     int n_dm = 0, hermi = 0, with_j = 0, with_k = 0, nstreams = 0, class_filter = -1;
     double cut = 0, fp32_tol = 0;
     size_t row_lds = 0;
     bool operator==(const GraphKey& o) const
     {
-        for (int i = 0; i < 5; ++i)
+        for (int i = 0; i < 6; ++i)
             if (bufs[i] != o.bufs[i]) return false;
         return dms == o.dms && vj == o.vj && vk == o.vk && n_dm == o.n_dm && hermi == o.hermi &&
                class_filter == o.class_filter &&
@@ -424,6 +426,10 @@ struct mjk_basis {
     double4* tW = nullptr;
     int *tpos = nullptr, *tstride = nullptr;
     double4 *rA = nullptr, *rAB = nullptr;
+    std::vector<JGroup> jgroups;     // J' by shell pair: the pair groups that have pairs and no f shells
+    std::vector<int> jgroup_of;      // group -> index in jgroups, -1: none
+    JGroup* d_jgroups = nullptr;
+    long long jtot = 0;              // elements of one density
     std::vector<int> seg;            // [(group * nmol + mol) * NBUCKET + bucket] -> first pair, group = class * NGT + type
     int* d_pmol = nullptr;           // molecule of every pair
     int* d_active = nullptr;         // per molecule: 0 skips its quartets (mjk_basis_set_active)
@@ -450,6 +456,8 @@ struct mjk_basis {
     // work buffers
     double *Dsph = nullptr, *Vj = nullptr, *Vk = nullptr;
     double *Dj = nullptr, *Dk = nullptr, *J = nullptr, *K = nullptr, *dmcond = nullptr;
+    double* Jp = nullptr;            // J' by shell pair, private copies
+    long long cap_jp = 0;
     long long cap_ds = 0, cap_vj = 0, cap_vk = 0, cap_dj = 0, cap_j = 0, cap_dk = 0, cap_k = 0, cap_cond = 0;
     unsigned long long* counters = nullptr;
     std::vector<void*> owned;
@@ -1248,6 +1256,27 @@ int build_basis(mjk_ctx* ctx, mjk_basis* b, double cutoff)
     b->q = qflat;
     flatten(b->seg);
     if ((rc = upload_pairs(&b->q))) return rc;
+    // J' by shell pair: component-major per pair group
+    b->jgroup_of.assign(NGROUP, -1);
+    for (int G = 0; G < NGROUP; ++G) {
+        const int p0 = b->seg[(size_t)G * nmol * NBUCKET], p1 = b->seg[(size_t)(G + 1) * nmol * NBUCKET];
+        int la = 0;
+        const int X = G / NGT, t = G % NGT;
+        while ((la + 1) * (la + 2) / 2 <= X) ++la;
+        if (p1 <= p0 || la > 2) continue;
+        JGroup g;
+        g.e0 = b->jtot;
+        g.p0 = p0;
+        g.n = p1 - p0;
+        g.la = la;
+        g.lb = X - la * (la + 1) / 2;
+        g.ca = group_ca(t);
+        g.cb = group_cb(t);
+        b->jgroup_of[G] = (int)b->jgroups.size();
+        b->jgroups.push_back(g);
+        b->jtot += (long long)g.n * g.ca * g.cb * ncart(g.la) * ncart(g.lb);
+    }
+    if ((rc = track_upload(b, b->jgroups, &b->d_jgroups))) return rc;
     b->pcost.assign(np + 1, 0);
     for (int p = 0; p < np; ++p) b->pcost[p + 1] = b->pcost[p] + b->h_nprim[p];
     {
@@ -1635,7 +1664,7 @@ void mjk_basis_destroy(mjk_basis* b)
     (void)hipStreamSynchronize(ctx->stream);
     free_tiles(b);
     for (void* p : b->owned) dfree(ctx, p);
-    double* work[] = {b->Dsph, b->Vj, b->Vk, b->Dj, b->Dk, b->J, b->K, b->dmcond};
+    double* work[] = {b->Dsph, b->Vj, b->Vk, b->Dj, b->Dk, b->J, b->K, b->Jp, b->dmcond};
     for (double* p : work) dfree(ctx, p);
     for (hipEvent_t e : b->pev) (void)hipEventDestroy(e);
     delete b;
@@ -1720,20 +1749,25 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     const int n_k = with_k ? (hermi == 1 ? n_dm : 2 * n_dm) : 0;
     const long long jcopy = (long long)std::max(n_j, 1) * b->slot_c;
     const long long kcopy = (long long)std::max(n_k, 1) * b->slot_c;
+    const long long jpcopy = (long long)n_j * b->jtot;   // J' by shell pair
     const bool need_cond = screen || fp32_tol > 0;
     // work buffers: Cartesian densities, private J'/K' copies, dm_cond
-    double *Dj, *Dk, *Jacc, *Kacc, *dmcond;
+    double *Dj, *Dk, *Jacc, *Kacc, *Jpair = nullptr, *dmcond;
     int ncopy = ctx->ncopy;
     if (!noalloc) {
         if ((rc = ensure(ctx, &b->Dj, b->cap_dj, jcopy))) return rc;
         if ((rc = ensure(ctx, &b->J, b->cap_j, ncopy * jcopy))) return rc;
         if ((rc = ensure(ctx, &b->Dk, b->cap_dk, kcopy))) return rc;
         if ((rc = ensure(ctx, &b->K, b->cap_k, ncopy * kcopy))) return rc;
+        if (jpcopy > 0) {
+            if ((rc = ensure(ctx, &b->Jp, b->cap_jp, ncopy * jpcopy))) return rc;
+            Jpair = b->Jp;
+        }
         if (need_cond && (rc = ensure(ctx, &b->dmcond, b->cap_cond, b->cond_total))) return rc;
         Dj = b->Dj, Dk = b->Dk, Jacc = b->J, Kacc = b->K, dmcond = b->dmcond;
     } else {
         // each buffer starts on a 256-byte boundary; as many accumulator copies
-        // as fit (at most the context's), at least one
+        // as fit (at most the context's), at least one; every J' in the arena
         auto up = [](long long n) { return (n + 31) / 32 * 32; };
         const long long cap = (long long)(MJK_NOALLOC_SCRATCH_BYTES / sizeof(double));
         auto need = [&](int nc) {
@@ -1762,7 +1796,8 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     // accumulators are cleared by a kernel, not a memset node.
     auto enqueue = [&](bool capture) -> int {
     if (!capture) HIPCHK(ctx, hipEventRecord(ctx->ev[0], st));
-    if (n_j && launch_zero(Jacc, ncopy * jcopy, st)) return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
+    if (n_j && (launch_zero(Jacc, ncopy * jcopy, st) || (Jpair && launch_zero(Jpair, ncopy * jpcopy, st))))
+        return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
     if (n_k && launch_zero(Kacc, ncopy * kcopy, st)) return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
     // (the 64-bit counters are cleared as doubles: both are all-zero bits)
     if (tally && launch_zero(reinterpret_cast<double*>(b->counters), 4 * NQCLASS_MAX, st))
@@ -1781,13 +1816,11 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     a.M.nsh = b->d_nsh;
     a.Dj = Dj;
     a.Dk = Dk;
-    a.J = Jacc;
     a.K = Kacc;
     a.slot = b->slot_c;
     a.n_j = n_j;
     a.n_k = n_k;
     a.ncopy = ncopy;
-    a.jcopy = jcopy;
     a.kcopy = kcopy;
     a.dm_cond = dmcond;
     a.cutoff = cut;
@@ -1852,6 +1885,21 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         a.bt_off = qc.bt_off;
         a.nbt = qc.nbt;
         a.diag = qc.GX == qc.GY;
+        // the row kernels without f shells accumulate J' by shell pair
+        const int jx = b->jgroup_of[qc.GX], jy = b->jgroup_of[qc.GY];
+        const bool jrow = qc.mode == 2 || row_choice(ctx, b, qc, n_j, n_k) == 1;
+        a.jpair = Jpair && jrow && jx >= 0 && jy >= 0;
+        a.J = a.jpair ? Jpair : Jacc;
+        a.jcopy = a.jpair ? jpcopy : jcopy;
+        a.jslot = a.jpair ? b->jtot : b->slot_c;
+        if (a.jpair) {
+            const JGroup &gx = b->jgroups[jx], &gy = b->jgroups[jy];
+            a.jb0 = gx.e0, a.jbn = gx.n, a.jbp0 = gx.p0;
+            a.jq0 = gy.e0, a.jqn = gy.n, a.jqp0 = gy.p0;
+        } else {
+            a.jb0 = a.jq0 = 0;
+            a.jbn = a.jbp0 = a.jqn = a.jqp0 = 0;
+        }
         a.counters = tally ? b->counters + 4 * c : nullptr;   // work tallies only on request
         // the row launches' size: one block per task, or the persistent grid
         int nrow_blocks = qc.nrt;
@@ -1908,8 +1956,29 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         HIPCHK(ctx, hipStreamWaitEvent(st, ctx->ev_join[i - 1], 0));
     }
     if (!capture) HIPCHK(ctx, hipEventRecord(ctx->ev[2], st));
+    if (launch_sum_copies(Kacc, n_k * b->slot_c, ncopy, kcopy, st) ||
+        launch_sum_copies(Jacc, n_j * b->slot_c, ncopy, jcopy, st))
+        return fail(ctx, MJK_EDEVICE, "accumulator sum launch failed");
+    if (Jpair) {
+        ScatterArgs sa;
+        sa.J = Jpair;
+        sa.jtot = b->jtot;
+        sa.n_j = n_j;
+        sa.ncopy = ncopy;
+        sa.jcopy = jpcopy;
+        sa.arena = Jacc;
+        sa.slot = b->slot_c;
+        sa.groups = b->d_jgroups;
+        sa.ngroup = (int)b->jgroups.size();
+        sa.cartA = b->cartA;
+        sa.cartB = b->cartB;
+        sa.pmol = b->d_pmol;
+        sa.dbase = b->d_dbase;
+        sa.ld = b->d_ld;
+        if (launch_jscatter(sa, st)) return fail(ctx, MJK_EDEVICE, "accumulator sum launch failed");
+    }
     if (launch_cart2sph(xform(b), b->maxnao, Jacc, Kacc, b->slot_c, n_dm, hermi, with_j, with_k, d_vj, d_vk,
-                        b->slot_s, ncopy, jcopy, kcopy, st))
+                        b->slot_s, st))
         return fail(ctx, MJK_EDEVICE, "output transform launch failed");
     if (!capture) HIPCHK(ctx, hipEventRecord(ctx->ev[3], st));
     return MJK_OK;
@@ -1922,8 +1991,8 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         key.dms = d_dms;
         key.vj = with_j ? d_vj : nullptr;
         key.vk = with_k ? d_vk : nullptr;
-        const void* bufs[5] = {Jacc, Kacc, Dj, Dk, dmcond};
-        for (int i = 0; i < 5; ++i) key.bufs[i] = bufs[i];
+        const void* bufs[6] = {Jacc, Kacc, Dj, Dk, dmcond, Jpair};
+        for (int i = 0; i < 6; ++i) key.bufs[i] = bufs[i];
         key.n_dm = n_dm;
         key.hermi = hermi;
         key.with_j = with_j;
