@@ -98,8 +98,8 @@ int nao_of(const std::vector<int>& bas, int nbas)
 
 // Upper estimate of the device bytes a request holds: primitive pairs (split
 // and merged representations), shell pairs, quartet task lists, the
-// Cartesian arenas (densities, the accumulator copies), dm_cond and, for an
-// RHF, the SCF state.
+// Cartesian arenas (densities, the accumulator copies), J' by shell pair (at
+// most an arena per copy), dm_cond and, for an RHF, the SCF state.
 size_t estimate_bytes(const Req& r)
 {
     double sp = 0, sp2 = 0;
@@ -117,7 +117,7 @@ size_t estimate_bytes(const Req& r)
     const double n = r.nao, nc = (double)ncart;
     const int ndm = std::max(r.n_dm, 1);
     double bytes = 48 * nprim_pairs + 160 * npairs + 16.0 * 55 * 16 * (npairs / 8 + 1) * 2;
-    bytes += 8.0 * (ndm * (3 + 2 * 8) * nc * nc + 3.0 * ndm * n * n + (double)nsh * nsh);
+    bytes += 8.0 * (ndm * (3 + 3 * 8) * nc * nc + 3.0 * ndm * n * n + (double)nsh * nsh);
     // the SCF state: 15 n^2 matrices, two histories of 8, the solver workspace
     // (at least 4 n^2 doubles and 32 MiB), small vectors
     if (r.kind == MJK_REQ_RHF) bytes += 8.0 * (15 + 2 * 8 + 4 + 1) * n * n + (double)(32 << 20);
