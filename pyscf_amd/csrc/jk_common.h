@@ -88,13 +88,15 @@ struct JKArgs {
     // f * (pairs of the group) + (q - first pair), so that lanes holding consecutive
     // kets add to consecutive addresses; else in the Cartesian arena.  MI355X, FP64
     // atomics of a wave: 23.6 G lane-adds/s to 64 scattered addresses, 163-181 G to
-    // 64 consecutive ones.
+    // 64 consecutive ones.  The row kernels add the bra's J'[a,b], once per block, to
+    // the arena Jb.
     double* J;
     long long jslot;
-    long long jq0, jb0;     // first element of the ket's and of the bra's pair group
+    long long jq0;          // first element of the ket's pair group
     int jpair;
     int jqn, jqp0;          // pairs and first pair of the ket's group
-    int jbn, jbp0;          // ... of the bra's group
+    double* Jb;             // Cartesian arena of J' (n_j slots of `slot` elements)
+    long long jbcopy;       // element stride between its copies
     double* K;              // accumulators K' (n_k slots), Cartesian arena
     long long slot;         // slot stride of the arenas (elements)
     int n_j;

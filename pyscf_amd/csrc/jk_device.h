@@ -121,15 +121,10 @@ __device__ __forceinline__ void atomic_add(double* p, double v)
     unsafeAtomicAdd(p, v);
 }
 
-// Element of a J' slot: component 0 of ket pair q (Cartesian offsets oc, od);
-// component f of bra pair p, by shell pair.
+// Element of a J' slot: component 0 of ket pair q (Cartesian offsets oc, od).
 __device__ __forceinline__ long long jket_at(const JKArgs& a, int q, long long base, int ld, int oc, int od)
 {
     return a.jpair ? a.jq0 + (q - a.jqp0) : base + (long long)oc * ld + od;
-}
-__device__ __forceinline__ long long jbra_at(const JKArgs& a, int f, int p)
-{
-    return a.jb0 + (long long)f * a.jbn + (p - a.jbp0);
 }
 
 // Load of read-only data at a wave-uniform address through the scalar cache
@@ -1702,9 +1697,7 @@ __global__ __launch_bounds__(256) void k_jk_row_gc(const JKArgs a)
         if (v == 0.0) continue;
         const int s = e / (NRA * NRB);
         const int ra = (e / NRB) % NRA, rb = e % NRB;
-        const int f = (((ra / G::NA) * CB + rb / G::NB) * G::NA + ra % G::NA) * G::NB + rb % G::NB;
-        atomic_add(a.J + cp * a.jcopy + s * a.jslot +
-                       (a.jpair ? jbra_at(a, f, p) : base + (long long)(oa + ra) * ld + ob + rb), v);
+        atomic_add(a.Jb + cp * a.jbcopy + s * a.slot + base + (long long)(oa + ra) * ld + ob + rb, v);
     }
     __syncthreads();   // the next task rewrites the LDS rows
     }

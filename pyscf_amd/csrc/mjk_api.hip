@@ -1816,6 +1816,8 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     a.M.nsh = b->d_nsh;
     a.Dj = Dj;
     a.Dk = Dk;
+    a.Jb = Jacc;
+    a.jbcopy = jcopy;
     a.K = Kacc;
     a.slot = b->slot_c;
     a.n_j = n_j;
@@ -1885,21 +1887,17 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         a.bt_off = qc.bt_off;
         a.nbt = qc.nbt;
         a.diag = qc.GX == qc.GY;
-        // the row kernels without f shells accumulate J' by shell pair
-        const int jx = b->jgroup_of[qc.GX], jy = b->jgroup_of[qc.GY];
-        const bool jrow = qc.mode == 2 || row_choice(ctx, b, qc, n_j, n_k) == 1;
-        a.jpair = Jpair && jrow && jx >= 0 && jy >= 0;
+        // the row kernels accumulate J' of kets without f shells by shell pair
+        const int rowk = qc.mode == 2 ? 0 : row_choice(ctx, b, qc, n_j, n_k);
+        const bool row_class = qc.mode == 2 || rowk > 0;
+        const int jy = b->jgroup_of[qc.GY];
+        a.jpair = Jpair && row_class && jy >= 0;
         a.J = a.jpair ? Jpair : Jacc;
         a.jcopy = a.jpair ? jpcopy : jcopy;
         a.jslot = a.jpair ? b->jtot : b->slot_c;
-        if (a.jpair) {
-            const JGroup &gx = b->jgroups[jx], &gy = b->jgroups[jy];
-            a.jb0 = gx.e0, a.jbn = gx.n, a.jbp0 = gx.p0;
-            a.jq0 = gy.e0, a.jqn = gy.n, a.jqp0 = gy.p0;
-        } else {
-            a.jb0 = a.jq0 = 0;
-            a.jbn = a.jbp0 = a.jqn = a.jqp0 = 0;
-        }
+        a.jq0 = a.jpair ? b->jgroups[jy].e0 : 0;
+        a.jqn = a.jpair ? b->jgroups[jy].n : 0;
+        a.jqp0 = a.jpair ? b->jgroups[jy].p0 : 0;
         a.counters = tally ? b->counters + 4 * c : nullptr;   // work tallies only on request
         // the row launches' size: one block per task, or the persistent grid
         int nrow_blocks = qc.nrt;
@@ -1915,8 +1913,6 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
             a.tlist = nullptr;
             a.ntask = 0;
         }
-        const int rowk = qc.mode == 2 ? 0 : row_choice(ctx, b, qc, n_j, n_k);
-        const bool row_class = qc.mode == 2 || rowk > 0;
         if (compact && row_class && qc.nrt > 0 &&
             launch_compact_rows(qc.rt, qc.nrt, b->d_pmol, b->d_active, b->d_tlist + qc.tl0, b->d_tctl + ROW_TCTL * c, st))
             return fail(ctx, MJK_EDEVICE, "task compaction launch failed");
