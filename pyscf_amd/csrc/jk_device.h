@@ -992,7 +992,9 @@ __attribute__((amdgpu_waves_per_eu(CoopShape<LA, LB, LC, LD>::WPE))) void k_jk_c
 #undef BLK
         __syncthreads();   // the block region is rewritten by the next quartet
     }
-    if (jab_lds) {
+    // (with every ket screened out there is nothing to flush, and no barrier
+    // stood between the clearing of sJab and here)
+    if (jab_lds && nq_blk) {
         const int cp = xcc_copy(a.ncopy);
         for (int s = 0; s < a.n_j; ++s) {
             double* V = a.J + cp * a.jcopy + s * a.jslot + base;
