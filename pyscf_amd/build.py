@@ -45,20 +45,23 @@ def ncart(l):
     return (l + 1) * (l + 2) // 2
 
 
-def jk_split(la, lb, lc, ld):
-    """Slices of a quartet class (same rule as jk_split in jk_device.h)."""
+SLICE_NF = 108   # most Cartesian components a lane holds
+
+
+def jk_slices(la, lb, lc, ld):
+    """Blocks of the a, b and c components of a quartet class, one slice kernel
+    each (same rule as jk_slices in jk_device.h, where its figures stand)."""
     na, nb, nc, nd = ncart(la), ncart(lb), ncart(lc), ncart(ld)
-    nf = na * nb * nc * nd
-    if nf <= 81:
-        return 1
-    if (la, lb, lc, ld) == (2, 1, 1, 1):     # 81 per lane: one wave per SIMD either way
-        return 2
-    for s in range(2, na + 1):
-        if na % s == 0 and nf // s <= 54:
-            return s
-    if nf // (na * nb) <= 54:
-        return na * nb
-    return na * nb * nc
+    return min((ka * kb * kc, -ka, -kb, (ka, kb, kc))
+               for ka in range(1, na + 1) if na % ka == 0
+               for kb in range(1, nb + 1) if nb % kb == 0
+               for kc in range(1, nc + 1) if nc % kc == 0
+               if na * nb * nc * nd // (ka * kb * kc) <= SLICE_NF)[-1]
+
+
+def jk_split(la, lb, lc, ld):
+    ka, kb, kc = jk_slices(la, lb, lc, ld)
+    return ka * kb * kc
 
 
 SLICES_PER_UNIT = 3
@@ -70,15 +73,13 @@ def nfunc(c):
 
 def use_row(c):
     """Classes that get the row kernel (one block per bra-pair task, K' rows
-    accumulated in LDS): at most 120 Cartesian components per quartet, or at
-    most 180 with at most 9 ket components (the J'[c,d] updates stay per
-    quartet), cut into at most 6 slices.  Measured on MI355X ((H2O)16 def2-SVP,
-    ms per launch): (ds|ds) row 0.18 / cooperative 0.97, (dd|ss) 0.12 / 0.64,
-    (dp|pp) 0.84 / 1.11; (dd|ds) 0.29 / 0.16 and, in def2-TZVP, (fs|dp)
-    2.41 / 2.04 stay cooperative."""
-    nf = nfunc(c)
-    nket = ncart(c[2]) * ncart(c[3])
-    return jk_split(*c) <= 6 and (nf <= 120 or (nf <= 180 and nket <= 9))
+    accumulated in LDS, one ket quartet per lane): at most six slices, or ten
+    with no f shell but the first.  Measured on MI355X (def2-TZVP chain of 876
+    AOs, ms per launch, row / cooperative kernel): (dp|dp) 4.9 / 13.2,
+    (dd|ds) 2.1 / 8.8, (fs|dp) 4.4 / 19.0, (fp|dp) 7.3 / 17.1, (fd|dp)
+    5.8 / 10.9, (fp|dd) 4.3 / 4.8; beyond the line (ff|pp) 3.9 / 3.6, (fp|fp)
+    6.4 / 6.5, (ff|fs) 3.0 / 2.4, (dd|dd) 2.2 / 1.1, (fd|dd) 4.2 / 3.3."""
+    return jk_split(*c) <= (10 if max(c[1:]) < 3 else 6)
 
 
 def use_row_m(c):
@@ -88,8 +89,7 @@ def use_row_m(c):
     Cartesian functions (13 to 20 rows) while their 10 A rows fit to 2000,
     cut into at most two slices.  Measured on MI355X (def2-TZVP chain, 1442
     AOs, ms per launch, this kernel / the fallback): (fp|ps) 38.8 / 116.5
-    cooperative; (fp|ds) 70.6 / 50.7 and (fd|ps) 67.3 / 53.6 (five slices
-    each) stay on the fallback."""
+    cooperative."""
     return use_row(c) and c[0] == 3 and c[1] >= 1 and jk_split(*c) <= 2
 
 
@@ -140,7 +140,7 @@ def gc_key(k):
     return ((((((la * 4 + lb) * 4 + lc) * 4 + ld) * 2 + ca - 1) * 2 + cb - 1) * 2 + cc - 1) * 2 + cd - 1
 
 
-ROW_TCTL = 8   # ints per class of the persistent row launches (jk_common.h): count + 7 slice counters
+ROW_TCTL = 12  # ints per class of the persistent row launches (jk_common.h): count + 11 slice counters
 
 
 def generate():
@@ -149,11 +149,12 @@ def generate():
         if use_row(c) and jk_split(*c) > ROW_TCTL - 1:
             raise RuntimeError('row class %s has more slices than persistent-launch counters' % (c,))
     files = []
-    head = '// generated by pyscf_amd/build.py\n#include "jk_device.h"\nnamespace mjk {\n'
+    head = head0 = '// generated by pyscf_amd/build.py\n#include "jk_device.h"\nnamespace mjk {\n'
     tail = '}  // namespace mjk\n'
     classes = quartet_classes()
     for c in classes:
         split = jk_split(*c)
+        head = head0 + 'static_assert(jk_split(%d, %d, %d, %d) == %d);\n' % (c + (split,))
         if use_coop(c):
             body = ('int launch_%s(int nb, const JKArgs& a, hipStream_t st)\n{\n'
                     '    return launch_jk_coop<%d, %d, %d, %d>(nb, a, st);\n}\n' % ((_name(c),) + c))
@@ -176,6 +177,7 @@ def generate():
                                  '{\n    return launch_jk_row<%d, %d, %d, %d, %d, %s>(nb, a, shmem, st);\n}\n'
                                  % ((tag, _name(c), sl) + c + (sl, rsh)))
                     files.append(_write('%s_%s%d.hip' % (_name(c), tag, u0), head + body + tail))
+    head = head0
     for c in classes:
         if use_row_m(c):
             split = jk_split(*c)
@@ -238,7 +240,7 @@ def generate():
     rcases = ''.join('    case %d: return launch_row_%s(nblocks, a, shmem, st);\n' % (key(c), _name(c))
                      for c in classes if use_row(c))
     coop = ''.join('    case %d: return 1;\n' % key(c) for c in classes if use_coop(c))
-    avail = ''.join('    case %d: return 1;\n' % key(c) for c in classes if use_row(c))
+    avail = ''.join('    case %d: return %d;\n' % (key(c), jk_split(*c)) for c in classes if use_row(c))
     mcases = ''.join('    case %d: return launch_rowm_%s(nblocks, a, shmem, st);\n' % (key(c), _name(c))
                      for c in classes if use_row_m(c))
     mavail = ''.join('    case %d: return 1;\n' % key(c) for c in classes if use_row_m(c))
@@ -255,7 +257,7 @@ def generate():
             'int coop_kernel(int la, int lb, int lc, int ld)\n{\n'
             '    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {\n' + coop +
             '    default: return 0;\n    }\n}\n'
-            'int row_kernel_available(int la, int lb, int lc, int ld)\n{\n'
+            'int row_kernel_slices(int la, int lb, int lc, int ld)\n{\n'
             '    switch (((la * 4 + lb) * 4 + lc) * 4 + ld) {\n' + avail +
             '    default: return 0;\n    }\n}\n'
             'int launch_jk_rows(int la, int lb, int lc, int ld, int nblocks, const JKArgs& a, size_t shmem, '

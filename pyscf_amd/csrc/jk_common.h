@@ -29,7 +29,7 @@ constexpr int LMAX = 3;                       // s, p, d, f
 constexpr int NPAIRCLASS = (LMAX + 1) * (LMAX + 2) / 2;
 constexpr int TILE = 8;                       // quartet tile: 8 bra x 8 ket pairs
 constexpr int ROW_MAXBUCKET = 32;             // primitive-count buckets a row-kernel block can hold
-constexpr int ROW_TCTL = 8;                   // ints per class of the persistent launches: count, 7 slice heads
+constexpr int ROW_TCTL = 12;                  // ints per class of the persistent launches: count, 11 slice heads
 
 __host__ __device__ constexpr int ncart(int l) { return (l + 1) * (l + 2) / 2; }
 __host__ __device__ constexpr int nsph(int l) { return 2 * l + 1; }

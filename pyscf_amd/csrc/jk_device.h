@@ -195,16 +195,36 @@ __device__ __forceinline__ void count_work(unsigned long long* c, bool alive, in
 // index stays a constant and the slice's integrals live in registers.  The
 // roots and the vertical recurrence are recomputed per slice.
 
-// Slice geometry: depth 0 = all components, 1 = a block of NA / SPLIT
-// consecutive a components (one a when SPLIT = NA), 2 = fixed (a, b),
-// 3 = fixed (a, b, c).
-template <int NA, int NB, int NC, int SPLIT>
-struct SliceShape {
-    static constexpr int depth = SPLIT == 1                      ? 0
-                                 : (SPLIT <= NA && NA % SPLIT == 0) ? 1
-                                 : SPLIT == NA * NB                 ? 2
-                                                                    : 3;
+// Slices of a quartet class: blocks of its a, b and c components, ka kb kc of
+// them, fewest with at most 108 components each (of equally few, the one that
+// cuts a most: an a block fixes powers of x, y, z that leave parts of the
+// recurrences out).  Every slice repeats the roots and the vertical
+// recurrence, so few large ones win although past 54 components a lane's
+// registers (to 512) leave one wave per SIMD.  MI355X, def2-TZVP chain of 876
+// AOs, row kernel, ms in s slices: (fp|ps) 90 components 5: 15.0, 2: 7.5,
+// 1: 6.1; (dp|dp) 324 6: 6.6, 3: 4.9, 2: 15.1 (162 each spill); (fs|dp) 180
+// 5: 7.8, 2: 4.4; (fp|dp) 540 10: 9.9, 5: 7.3; (fp|pp) 270 5: 8.8, 2: 8.8,
+// 3 blocks of c: 7.8.
+constexpr int SLICE_NF = 108;
+struct Slices {
+    int ka, kb, kc;
 };
+__host__ __device__ constexpr Slices jk_slices(int la, int lb, int lc, int ld)
+{
+    const int na = ncart(la), nb = ncart(lb), nc = ncart(lc), nf = na * nb * nc * ncart(ld);
+    for (int n = 1;; ++n) {
+        if (nf > n * SLICE_NF) continue;
+        for (int ka = na; ka >= 1; --ka)
+            for (int kb = nb; kb >= 1; --kb)
+                if (na % ka == 0 && nb % kb == 0 && n % (ka * kb) == 0 && nc % (n / (ka * kb)) == 0)
+                    return {ka, kb, n / (ka * kb)};
+    }
+}
+__host__ __device__ constexpr int jk_split(int la, int lb, int lc, int ld)
+{
+    const Slices s = jk_slices(la, lb, lc, ld);
+    return s.ka * s.kb * s.kc;
+}
 
 struct QuartetCtx {
     int p, q, mol;
@@ -272,13 +292,11 @@ __device__ __forceinline__ double wave_sum_last(double v)
 template <int LA, int LB, int LC, int LD, int SPLIT, int S>
 struct SliceRange {
     static constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-    static constexpr int DEPTH = SliceShape<NA, NB, NC, SPLIT>::depth;
-    static constexpr int IA0 = DEPTH == 0 ? 0 : DEPTH == 1 ? S * (NA / SPLIT) : DEPTH == 2 ? S / NB : S / (NB * NC);
-    static constexpr int IA1 = DEPTH == 0 ? NA : DEPTH == 1 ? IA0 + NA / SPLIT : IA0 + 1;
-    static constexpr int IB0 = DEPTH <= 1 ? 0 : DEPTH == 2 ? S % NB : (S / NC) % NB;
-    static constexpr int IB1 = DEPTH <= 1 ? NB : IB0 + 1;
-    static constexpr int IC0 = DEPTH <= 2 ? 0 : S % NC;
-    static constexpr int IC1 = DEPTH <= 2 ? NC : IC0 + 1;
+    static constexpr Slices K = SPLIT == 1 ? Slices{1, 1, 1} : jk_slices(LA, LB, LC, LD);
+    static_assert(SPLIT == K.ka * K.kb * K.kc && S < SPLIT);
+    static constexpr int IA0 = S / (K.kb * K.kc) * (NA / K.ka), IA1 = IA0 + NA / K.ka;
+    static constexpr int IB0 = S / K.kc % K.kb * (NB / K.kb), IB1 = IB0 + NB / K.kb;
+    static constexpr int IC0 = S % K.kc * (NC / K.kc), IC1 = IC0 + NC / K.kc;
     static constexpr int MA = IA1 - IA0, MB = IB1 - IB0, MC = IC1 - IC0;
     static constexpr int NFL = MA * MB * MC * ND;
 };
@@ -361,8 +379,9 @@ __device__ __forceinline__ void add_root(const PrimQuartet& m, double rx, double
 
 // Contracted Cartesian block of one quartet restricted to slice S, times
 // the quartet's degeneracy factor, in FP64 (recurrences in precision R).
-// RSH: the kernel also evaluates the range-separated operators (a.omega != 0).
-template <int LA, int LB, int LC, int LD, int SPLIT, int S, typename R, bool UNIFORM_BRA = false, bool RSH = false,
+// RSH: 0 the Coulomb operator, 1 the range-separated operators (a.omega != 0),
+// 2 either.
+template <int LA, int LB, int LC, int LD, int SPLIT, int S, typename R, bool UNIFORM_BRA = false, int RSH = 0,
           bool LT = false>
 __device__ __forceinline__ void eri_slice(const JKArgs& a, const QuartetCtx& c,
                                           double (&gd)[SliceRange<LA, LB, LC, LD, SPLIT, S>::NFL])
@@ -380,7 +399,7 @@ __device__ __forceinline__ void eri_slice(const JKArgs& a, const QuartetCtx& c,
     for (int ib = 0; ib < c.npb; ++ib) {
         const double4 Pp = UNIFORM_BRA ? uload(a.P.ppP + c.pb0 + ib) : a.P.ppP[c.pb0 + ib];
         const double2 Kp = UNIFORM_BRA ? uload(a.P.ppK + c.pb0 + ib) : a.P.ppK[c.pb0 + ib];
-        if (RSH && a.omega != 0.0) {   // range-separated operator, one ket primitive at a time
+        if (RSH == 1 || (RSH == 2 && a.omega != 0.0)) {   // range-separated operator, one ket primitive at a time
             for (int ik = 0; ik < c.npk; ++ik) {
                 double T;
                 const int t0 = c.tq + ik * c.ts;
@@ -447,7 +466,7 @@ __device__ __forceinline__ void quartet_slice(const JKArgs& a, const QuartetCtx&
     constexpr int IA0 = SR::IA0, IA1 = SR::IA1, IB0 = SR::IB0, IB1 = SR::IB1, IC0 = SR::IC0, IC1 = SR::IC1;
     constexpr int MA = SR::MA, MB = SR::MB, MC = SR::MC;
     double gd[SR::NFL];
-    eri_slice<LA, LB, LC, LD, SPLIT, S, R, false, true>(a, c, gd);
+    eri_slice<LA, LB, LC, LD, SPLIT, S, R, false, 2>(a, c, gd);
 
     const long long base = a.M.dbase[c.mol];
     const int ld = a.M.ld[c.mol];
@@ -1018,22 +1037,6 @@ int launch_jk_coop(int nblocks, const JKArgs& a, hipStream_t st)
     return (int)hipGetLastError();
 }
 
-// Number of slices for a class: keep <= ~54 components per lane.
-__host__ __device__ constexpr int jk_split(int la, int lb, int lc, int ld)
-{
-    const int na = ncart(la), nb = ncart(lb), nc = ncart(lc), nd = ncart(ld);
-    const int nf = na * nb * nc * nd;
-    if (nf <= 81) return 1;
-    // (dp|pp): 81 per lane; at 54 its registers already exceeded 256 (one wave
-    // per SIMD), so the third slice only repeated the recurrences: C30H62
-    // cc-pVDZ class 3.40 -> 2.40 ms on MI355X (384 registers, no spills)
-    if (la == 2 && lb == 1 && lc == 1 && ld == 1) return 2;
-    for (int s = 2; s <= na; ++s)   // fewest blocks of a components with at most 54 components each
-        if (na % s == 0 && nf / s <= 54) return s;
-    if (nf / (na * nb) <= 54) return na * nb;
-    return na * nb * nc;
-}
-
 template <int LA, int LB, int LC, int LD, int S>
 int launch_jk_slice(int nblocks, const JKArgs& a, hipStream_t st)
 {
@@ -1077,7 +1080,7 @@ __device__ __forceinline__ void row_digest(const JKArgs& a, const QuartetCtx& c,
     constexpr int IA0 = SR::IA0, IA1 = SR::IA1, IB0 = SR::IB0, IB1 = SR::IB1, IC0 = SR::IC0, IC1 = SR::IC1;
     constexpr int MA = SR::MA, MB = SR::MB, MC = SR::MC;
     double gd[SR::NFL];
-    eri_slice<LA, LB, LC, LD, SPLIT, S, R, true, RSH, RowRys<LA, LB, LC, LD>::lds>(a, c, gd);
+    eri_slice<LA, LB, LC, LD, SPLIT, S, R, true, RSH ? 1 : 0, RowRys<LA, LB, LC, LD>::lds>(a, c, gd);
     const int oc = c.qvalid ? a.P.cartA[c.q] : 0, od = c.qvalid ? a.P.cartB[c.q] : 0;
     const int lane = threadIdx.x & 63;
     for (int s = 0; s < a.n_j; ++s) {

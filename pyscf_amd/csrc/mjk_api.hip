@@ -44,7 +44,7 @@
 namespace mjk {
 int launch_jk(int la, int lb, int lc, int ld, int nblocks, const JKArgs& a, hipStream_t st);
 int launch_jk_rows(int la, int lb, int lc, int ld, int nblocks, const JKArgs& a, size_t shmem, hipStream_t st);
-int row_kernel_available(int la, int lb, int lc, int ld);
+int row_kernel_slices(int la, int lb, int lc, int ld);   // 0: no row kernel
 int launch_jk_rows_gc(int la, int lb, int lc, int ld, int ca, int cb, int cc, int cd, int nblocks, const JKArgs& a,
                       size_t shmem, hipStream_t st);
 int row_gc_available(int la, int lb, int lc, int ld, int ca, int cb, int cc, int cd);
@@ -598,12 +598,22 @@ int build_tiles(mjk_basis* b, double cutoff)
             if ((rc = upload(ctx, btm, &qc.bt_mol))) return rc;
             if ((rc = upload(ctx, off, &qc.bt_off))) return rc;
         }
+        // A sliced row kernel (one quartet per lane, every slice a pass over the
+        // class) needs quartets to fill its lanes; below about 30 000 per slice
+        // the cooperative kernel (one quartet per block) is done before a pass's
+        // latency is over.  MI355X, ms, row / cooperative: (dd|ds) in 2 slices
+        // 28 k quartets 0.23 / 0.22, 130 k 0.35 / 0.64; (dd|pp) in 3 32 k 0.44 /
+        // 0.30, 74 k 0.67 / 0.57, 288 k 0.74 / 1.40; (dd|dp) in 6 65 k 0.70 /
+        // 0.53, 136 k 0.75 / 0.89; (fd|dp) in 10 61 k 1.27 / 0.82, 1.1 M 5.8 /
+        // 10.9.  A tuning entry may ask for either.
+        const bool merged = qc.ca * qc.cb * qc.cc * qc.cd > 1;
+        const int slices = merged ? 1 : row_kernel_slices(qc.la, qc.lb, qc.lc, qc.ld);
+        const bool few = slices > 1 && qc.kernel_pref != 1 && est_q < 3.0e4 * slices;
         // Row-kernel tasks: the same Schwarz prefixes per bra pair, cut into
         // chunks of about equal primitive-quartet count (the kets' primitive
         // counts differ up to a hundredfold).
-        if (qc.nbt > 0 && (qc.ca * qc.cb * qc.cc * qc.cd > 1
-                              ? row_gc_available(qc.la, qc.lb, qc.lc, qc.ld, qc.ca, qc.cb, qc.cc, qc.cd)
-                              : row_kernel_available(qc.la, qc.lb, qc.lc, qc.ld))) {
+        if (qc.nbt > 0 && !few &&
+            (merged ? row_gc_available(qc.la, qc.lb, qc.lc, qc.ld, qc.ca, qc.cb, qc.cc, qc.cd) : slices)) {
             std::vector<int2> rr;
             std::vector<int> bra;
             long long cost_all = 0;
