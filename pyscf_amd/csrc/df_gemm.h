@@ -29,4 +29,11 @@ int df_y(const double* B, const double* Xp, int nao, int naux, int ncol, double*
 size_t df_xp_size(int nao, int ncol);
 int df_pad_x(const double* src, long long sl, long long so, int nao, int ncol, double* Xp, hipStream_t st);
 
+// Cholesky factor of a symmetric positive definite n x n matrix (both triangles
+// given) into its lower triangle, column-major; the strict upper triangle is
+// left undefined.  info (zeroed by the caller): first row whose pivot is not
+// positive, from 1.  tmp: CHOL_NB^2 doubles.
+constexpr int CHOL_NB = 32;
+int df_potrf(double* A, int n, double* tmp, int* info, hipStream_t st);
+
 }  // namespace mjk

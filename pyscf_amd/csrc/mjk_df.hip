@@ -5,7 +5,7 @@
 //   * (P|Q) and (ij|P) by the Rys kernels of df_device.h into staging
 //     matrices with Cartesian auxiliary columns, then the auxiliary index to
 //     spherical functions (k_df_auxsph);
-//   * (P|Q) = L L^T (rocsolver_dpotrf), B = L^-1 (P|ij) (rocblas_dtrsm); when
+//   * (P|Q) = L L^T (df_potrf), B = L^-1 (P|ij) (rocblas_dtrsm); when
 //     the factorisation fails, B = (V w^-1/2)^T (P|ij) over the eigenpairs of
 //     (P|Q) with w above lindep, as the reference falls back.
 //   B stays in HBM as a column-major (naux x nao^2) matrix: for every orbital
@@ -17,8 +17,8 @@
 //     row i), then K = B^T Y over (P, l): K_ik = sum_Pl B_k[P,l] Y_i[P,l] =
 //     sum_P (B_P D B_P)_ik;
 //   * K of occupied orbitals X (D = X X^T): Y_i = B_i X, K = Y^T Y.
-// Both K products on the FP64 matrix cores (mjk_dfgemm.hip); the fit on
-// rocBLAS/rocSOLVER; everything on the context's stream, FP64 throughout.
+// Both K products on the FP64 matrix cores (mjk_dfgemm.hip), also the
+// Cholesky factor; the fit's solve and eigenvectors on rocBLAS/rocSOLVER; everything on the context's stream, FP64 throughout.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
@@ -83,21 +83,47 @@ void c2s_rows(std::vector<double>& tab)
 
 // B[row][P] = sum_c tab[l][m][c] S[row][col0[l] + c n[l] + u], per final auxiliary function
 // P = {l, m, u}; rows x naux outputs
-__global__ void k_df_auxsph(const double* __restrict__ S, long long lds, double* __restrict__ B, long long rows,
-                            int naux, const int4* __restrict__ map, const long long* __restrict__ col0,
-                            const int* __restrict__ ngrp, const double* __restrict__ tab)
+// Bandwidth-bound (S once, B once); a block takes 256 functions of AUXSPH_ROWS
+// rows, so that the lookups and the table serve them all and their loads are in
+// flight together.  MI355X, 900 functions of 5 10^4 orbital pairs: 0.35 ms; one
+// output per thread with a 64-bit division to find it 0.52.
+constexpr int AUXSPH_ROWS = 8;
+__global__ __launch_bounds__(256) void k_df_auxsph(const double* __restrict__ S, long long lds,
+                                                   double* __restrict__ B, long long rows, int naux, int ntile,
+                                                   const int4* __restrict__ map, const long long* __restrict__ col0,
+                                                   const int* __restrict__ ngrp, const double* __restrict__ tab)
 {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= rows * naux) return;
-    const long long row = t / naux;
-    const int P = (int)(t % naux);
+    const long long row0 = (long long)(blockIdx.x / ntile) * AUXSPH_ROWS;
+    const int P = blockIdx.x % ntile * 256 + threadIdx.x;
+    if (P >= naux) return;
     const int4 m = map[P];   // {l, m, unit in group, 0}
     const int l = m.x, nc = (l + 1) * (l + 2) / 2;
-    const double* s = S + row * lds + col0[l] + m.z;
+    const long long sc = ngrp[l];
+    const double* s[AUXSPH_ROWS];
+    double v[AUXSPH_ROWS];
+#pragma unroll
+    for (int r = 0; r < AUXSPH_ROWS; ++r) {   // (rows past the end read the last one and are not stored)
+        s[r] = S + min(row0 + r, rows - 1) * lds + col0[l] + m.z;
+        v[r] = 0.0;
+    }
     const double* tr = tab + (l * 9 + m.y) * 15;
-    double v = 0.0;
-    for (int c = 0; c < nc; ++c) v += tr[c] * s[(long long)c * ngrp[l]];
-    B[row * naux + P] = v;
+    for (int c = 0; c < nc; ++c) {
+        const double w = tr[c];
+#pragma unroll
+        for (int r = 0; r < AUXSPH_ROWS; ++r) v[r] += w * s[r][c * sc];
+    }
+#pragma unroll
+    for (int r = 0; r < AUXSPH_ROWS; ++r)
+        if (row0 + r < rows) B[(row0 + r) * naux + P] = v[r];
+}
+
+int launch_auxsph(const double* S, long long lds, double* B, long long rows, int naux, const int4* map,
+                  const long long* col0, const int* ngrp, const double* tab, hipStream_t st)
+{
+    const int ntile = (naux + 255) / 256;
+    const long long nb = (rows + AUXSPH_ROWS - 1) / AUXSPH_ROWS * ntile;
+    k_df_auxsph<<<(unsigned)nb, 256, 0, st>>>(S, lds, B, rows, naux, ntile, map, col0, ngrp, tab);
+    return (int)hipGetLastError();
 }
 
 // J of one density from the fitted tensor, two passes over the lower-triangle
@@ -388,12 +414,8 @@ int build(mjk_ctx* ctx, mjk_df* df, const int* atm, int natm, const int* bas, in
             if (launch_int3c(li, 0, lk, true, a, st)) return ctx_fail(ctx, MJK_EDEVICE, "(P|Q) launch failed");
         }
     }
-    {
-        const long long n = (long long)naux * naux;
-        k_df_auxsph<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(S2, ncol, df->j2c, naux, naux, d_map, d_col0, d_gn,
-                                                                 d_tab);
-        HC(ctx, hipGetLastError());
-    }
+    if (launch_auxsph(S2, ncol, df->j2c, naux, naux, d_map, d_col0, d_gn, d_tab, st))
+        return ctx_fail(ctx, MJK_EDEVICE, "auxiliary transform launch failed");
     // (ij|P)
     if ((rc = mjk_device_alloc(ctx, sizeof(double) * (size_t)nn * ncol, (void**)&S3))) return rc;
     tmp.ptrs.push_back(S3);
@@ -431,12 +453,8 @@ int build(mjk_ctx* ctx, mjk_df* df, const int* atm, int natm, const int* bas, in
             }
         }
     if ((rc = mjk_device_alloc(ctx, sizeof(double) * (size_t)nn * naux, (void**)&df->B))) return rc;
-    {
-        const long long n = nn * naux;
-        k_df_auxsph<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(S3, ncol, df->B, nn, naux, d_map, d_col0, d_gn,
-                                                                 d_tab);
-        HC(ctx, hipGetLastError());
-    }
+    if (launch_auxsph(S3, ncol, df->B, nn, naux, d_map, d_col0, d_gn, d_tab, st))
+        return ctx_fail(ctx, MJK_EDEVICE, "auxiliary transform launch failed");
     HC(ctx, hipStreamSynchronize(st));
     (void)mjk_device_free(ctx, S3);
     tmp.ptrs.back() = nullptr;
@@ -463,7 +481,6 @@ int build(mjk_ctx* ctx, mjk_df* df, const int* atm, int natm, const int* bas, in
     RB(ctx, rocblas_start_device_memory_size_query(h));
     {
         const double one = 1.0;
-        (void)rocsolver_dpotrf(h, rocblas_fill_lower, naux, L, naux, info);
         (void)rocsolver_dsyevd(h, rocblas_evect_original, rocblas_fill_upper, naux, L, naux, wv, wv + naux, info);
         (void)rocblas_dtrsm(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none, rocblas_diagonal_non_unit,
                             naux, (rocblas_int)nn, &one, L, naux, df->B, naux);
@@ -471,7 +488,11 @@ int build(mjk_ctx* ctx, mjk_df* df, const int* atm, int natm, const int* bas, in
     RB(ctx, rocblas_stop_device_memory_size_query(h, &need));
     if ((rc = workspace(df, h, need))) return rc;
     RB(ctx, rocblas_set_pointer_mode(h, rocblas_pointer_mode_host));
-    RB(ctx, rocsolver_dpotrf(h, rocblas_fill_lower, naux, L, naux, info));
+    double* dtmp = nullptr;
+    if ((rc = mjk_device_alloc(ctx, sizeof(double) * CHOL_NB * CHOL_NB, (void**)&dtmp))) return rc;
+    tmp.ptrs.push_back(dtmp);
+    HC(ctx, hipMemsetAsync(info, 0, sizeof(rocblas_int), st));
+    if (df_potrf(L, naux, dtmp, info, st)) return ctx_fail(ctx, MJK_EDEVICE, "Cholesky launch failed");
     rocblas_int hinfo = 0;
     HC(ctx, hipMemcpyAsync(&hinfo, info, sizeof(hinfo), hipMemcpyDeviceToHost, st));
     HC(ctx, hipStreamSynchronize(st));

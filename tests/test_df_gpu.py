@@ -191,3 +191,26 @@ def test_exchange_matrix_core_tiles(size):
     vj, vk = df.get_jk(d, dm, 0)
     k0 = numpy.einsum('pij,jk,pkl->il', b, dm, b, optimize=True)
     assert abs(vk - k0).max() <= 1e-12 * abs(k0).max()
+
+
+@pytest.mark.parametrize('n', [1, 31, 32, 33, 97, 161])
+def test_fit_factor_block_edges(n):
+    """The blocked Cholesky factor of (P|Q) at the edges of its 32-column blocks
+    and 64-row tiles, and the auxiliary transform at the ends of its row groups:
+    n atoms with one s function each.  Both fits are backward stable, so they
+    differ by less than 8 n eps cond(L) of the largest element."""
+    import scipy.linalg
+    g = numpy.array([(i % 6, i // 6 % 6, i // 36) for i in range(n)]) * 3.0
+    g += numpy.random.default_rng(n).uniform(-0.4, 0.4, g.shape)
+    mol = gto.M(atom=[('H', tuple(x)) for x in g], unit='bohr', basis={'H': [[0, (0.5, 1.0)]]}, spin=n % 2)
+    aux = {'H': [[0, (0.8, 1.0)]]}
+    d = df.DF(mol, aux)
+    d.lindep = -1.0
+    raw = d.build().cderi().reshape(n, -1)
+    j2 = numpy.empty((n, n))
+    d.engine.check(d.engine.lib.mjk_df_fetch(d.engine.handle, d.handle, 0, j2.ctypes.data_as(lib.ctypes.c_void_p)),
+                   'mjk_df_fetch')
+    L = numpy.linalg.cholesky(j2)
+    ref = scipy.linalg.solve_triangular(L, raw, lower=True)
+    fit = df.DF(mol, aux).build().cderi().reshape(n, -1)
+    assert abs(fit - ref).max() <= 8 * n * 2.3e-16 * numpy.linalg.cond(L) * abs(ref).max()
