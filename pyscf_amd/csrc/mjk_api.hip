@@ -27,6 +27,7 @@
 #include <sstream>
 #include <dlfcn.h>
 #include <map>
+#include <set>
 #include <tuple>
 #include <mutex>
 #include <shared_mutex>
@@ -219,6 +220,7 @@ struct mjk_ctx {
     std::string err;
     double* rys = nullptr;
     std::map<void*, size_t> allocs;
+    std::set<mjk_basis*> bases;           // of this context, not yet destroyed
     std::recursive_mutex mu;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     // extra streams (default priority) on which the quartet classes of a build
@@ -258,15 +260,27 @@ int fail(mjk_ctx* ctx, int code, const char* fmt, ...)
         if (e_ != hipSuccess) return fail(ctx, MJK_EDEVICE, "%s failed: %s", #x, hipGetErrorString(e_)); \
     } while (0)
 
-int dalloc(mjk_ctx* ctx, size_t bytes, void** p)
+// Frees the J' accumulators by shell pair of the context's bases (a build goes
+// without them where they do not fit); false: there were none.
+bool drop_jpairs(mjk_ctx* ctx);
+
+// Device memory within the budget; must: the accumulators by shell pair make
+// room where it is short.
+int dalloc(mjk_ctx* ctx, size_t bytes, void** p, bool must = true)
 {
     *p = nullptr;
     if (bytes == 0) return MJK_OK;
+    if (ctx->used + bytes > ctx->budget && must) (void)drop_jpairs(ctx);
     if (ctx->used + bytes > ctx->budget)
         return fail(ctx, MJK_ENOMEM, "HBM budget exceeded: need %zu more bytes, %zu of %zu in use", bytes,
                     ctx->used.load(), ctx->budget);
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) return fail(ctx, MJK_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess && must && drop_jpairs(ctx)) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // or the next launch's check would report it
+        *p = nullptr;
+        return fail(ctx, MJK_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    }
     ctx->used += bytes;
     ctx->allocs[*p] = bytes;
     return MJK_OK;
@@ -1384,16 +1398,29 @@ std::vector<char> classes_to_run(const mjk_ctx* ctx, const mjk_basis* b, int n_j
     return run;
 }
 
-int ensure(mjk_ctx* ctx, double** p, long long& cap, long long need)
+int ensure(mjk_ctx* ctx, double** p, long long& cap, long long need, bool must = true)
 {
     if (need <= cap && *p) return MJK_OK;
     dfree(ctx, *p);
     *p = nullptr;
     cap = 0;
-    int rc = dalloc(ctx, sizeof(double) * std::max(need, 1LL), (void**)p);
+    int rc = dalloc(ctx, sizeof(double) * std::max(need, 1LL), (void**)p, must);
     if (rc) return rc;
     cap = need;
     return MJK_OK;
+}
+
+bool drop_jpairs(mjk_ctx* ctx)
+{
+    bool any = false;
+    for (mjk_basis* b : ctx->bases) {
+        if (!b->Jp) continue;
+        dfree(ctx, b->Jp);
+        b->Jp = nullptr;
+        b->cap_jp = 0;
+        any = true;
+    }
+    return any;
 }
 
 }  // namespace
@@ -1632,6 +1659,7 @@ int mjk_basis_upload_batch(mjk_ctx* ctx, int nmol, const int* natm, const int* n
     *out = nullptr;
     mjk_basis* b = new mjk_basis();
     b->ctx = ctx;
+    ctx->bases.insert(b);
     b->nmol = nmol;
     b->mols.resize(nmol);
     int rc = MJK_OK;
@@ -1677,6 +1705,7 @@ void mjk_basis_destroy(mjk_basis* b)
     double* work[] = {b->Dsph, b->Vj, b->Vk, b->Dj, b->Dk, b->J, b->K, b->Jp, b->dmcond};
     for (double* p : work) dfree(ctx, p);
     for (hipEvent_t e : b->pev) (void)hipEventDestroy(e);
+    ctx->bases.erase(b);
     delete b;
 }
 
@@ -1769,11 +1798,9 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         if ((rc = ensure(ctx, &b->J, b->cap_j, ncopy * jcopy))) return rc;
         if ((rc = ensure(ctx, &b->Dk, b->cap_dk, kcopy))) return rc;
         if ((rc = ensure(ctx, &b->K, b->cap_k, ncopy * kcopy))) return rc;
-        if (jpcopy > 0) {
-            if ((rc = ensure(ctx, &b->Jp, b->cap_jp, ncopy * jpcopy))) return rc;
-            Jpair = b->Jp;
-        }
         if (need_cond && (rc = ensure(ctx, &b->dmcond, b->cap_cond, b->cond_total))) return rc;
+        // after all that the build must have: where it does not fit, every J' goes to the arena
+        if (jpcopy > 0 && ensure(ctx, &b->Jp, b->cap_jp, ncopy * jpcopy, false) == MJK_OK) Jpair = b->Jp;
         Dj = b->Dj, Dk = b->Dk, Jacc = b->J, Kacc = b->K, dmcond = b->dmcond;
     } else {
         // each buffer starts on a 256-byte boundary; as many accumulator copies

@@ -385,3 +385,39 @@ def test_sliced_row_classes_match_cooperative(omega):
         for i in (0, 1):
             d = abs(out[1, k][i] - out[2, k][i]).max()
             assert d < 1e-12 * max(1.0, scale[i]), (k, i, d)
+
+
+def test_builds_without_room_for_pair_accumulators():
+    """The J' accumulators by shell pair are taken only where they fit: one byte
+    of budget less than a build took, it runs without them, and an allocation
+    that needs their room gets it.  The same sums in another order: 1e-12 of the
+    largest element."""
+    import ctypes
+    mol = gto.M(atom=workloads.water_cluster(2, shape=(2, 1, 1)), basis='cc-pvdz')
+    dms = numpy.random.default_rng(5).standard_normal((2, mol.nao_nr(), mol.nao_nr()))
+
+    def build(eng, b):
+        jk = b.get_jk(dms, 0, True, True, 1e-13)
+        return jk, eng.hbm_used()
+
+    eng = _vhf.Engine()
+    ref, full = build(eng, eng.upload(mol._atm, mol._bas, mol._env, 1e-13))
+    eng1 = _vhf.Engine(hbm_budget=full - 1)
+    b1 = eng1.upload(mol._atm, mol._bas, mol._env, 1e-13)
+    out = [build(eng1, b1) for _ in range(3)]
+    eng2 = _vhf.Engine(hbm_budget=full)
+    b2 = eng2.upload(mol._atm, mol._bas, mol._env, 1e-13)
+    out += [build(eng2, b2) for _ in range(3)]
+    assert [u for _, u in out[3:]] == [full] * 3
+    lean = out[0][1]
+    assert lean < full and [u for _, u in out[:3]] == [lean] * 3
+    p = ctypes.c_void_p()
+    eng2.check(eng2.lib.mjk_device_alloc(eng2.handle, full - lean, ctypes.byref(p)), 'mjk_device_alloc')
+    assert eng2.hbm_used() == full
+    out += [build(eng2, b2) for _ in range(3)]
+    eng2.check(eng2.lib.mjk_device_free(eng2.handle, p), 'mjk_device_free')
+    out += [build(eng2, b2) for _ in range(3)]
+    assert out[-1][1] == full
+    for jk, _ in out:
+        for x, r in zip(jk, ref):
+            assert abs(x - r).max() <= 1e-12 * abs(r).max()
