@@ -53,10 +53,8 @@ struct mjk_df {
     size_t caprho = 0;
     void* ws = nullptr;
     size_t capws = 0;
-    double* X = nullptr;       // padded orbitals (or density) of the half transform
-    size_t capX = 0;
-    double* part = nullptr;    // slices of the exchange product
-    size_t cappart = 0;
+    double* kbuf = nullptr;    // scratch of the exchange where `ws` is too small for it
+    size_t capk = 0;
 };
 
 namespace {
@@ -564,10 +562,20 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
     if (with_k) {
         const long long kin = (long long)naux * ncol;
         const TnPlan plan = df_tn_plan(nao, std::max(kin, 1LL), d_orbo != nullptr);
+        // scratch: padded orbitals (or density) of the half transform, slices of
+        // the product.  The fit's workspace (32 MiB, or a copy of B for the
+        // solve) is idle now, on this stream and larger at all usual sizes.
+        const size_t nx = df_xp_size(nao, ncol);
+        double *X = nullptr, *part = nullptr;
         if (ncol > 0) {
             if ((rc = grow(ctx, &df->Y, &df->capY, (size_t)nao * kin))) return rc;
-            if ((rc = grow(ctx, &df->X, &df->capX, df_xp_size(nao, ncol)))) return rc;
-            if ((rc = grow(ctx, &df->part, &df->cappart, plan.ws))) return rc;
+            if (sizeof(double) * (nx + plan.ws) <= df->capws)
+                X = (double*)df->ws;
+            else if ((rc = grow(ctx, &df->kbuf, &df->capk, nx + plan.ws)))
+                return rc;
+            else
+                X = df->kbuf;
+            part = X + nx;
         }
         for (int k = 0; k < n_dm; ++k) {
             double* K = d_vk + (size_t)k * nn;
@@ -578,12 +586,12 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
             // Y_i (naux x ncol) = B_i (naux x nao) M, M = D or X, row-major or (orbo_colmajor) column-major
             const double* M = d_orbo ? d_orbo + (size_t)k * nao * nocc : d_dms + (size_t)k * nn;
             const bool cm = d_orbo && orbo_colmajor;
-            if (df_pad_x(M, cm ? 1 : ncol, cm ? nao : 1, nao, ncol, df->X, st) ||
-                df_y(df->B, df->X, nao, naux, ncol, df->Y, st))
+            if (df_pad_x(M, cm ? 1 : ncol, cm ? nao : 1, nao, ncol, X, st) ||
+                df_y(df->B, X, nao, naux, ncol, df->Y, st))
                 return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: half-transform launch failed");
             // K = Y^T Y over (P, o), symmetric; or K (row-major) = B^T Y over
             // (P, l): column-major C(k, i) = K[i][k]
-            if (df_tn(plan, d_orbo ? df->Y : df->B, df->Y, nao, kin, d_orbo != nullptr, df->part, K, st))
+            if (df_tn(plan, d_orbo ? df->Y : df->B, df->Y, nao, kin, d_orbo != nullptr, part, K, st))
                 return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: exchange product launch failed");
         }
     }
@@ -597,7 +605,7 @@ void release(mjk_df* df)
         (void)hipStreamSynchronize(mjk_internal::ctx_stream(df->ctx));
         if (rocblas_handle h = (rocblas_handle)mjk_internal::ctx_blas(df->ctx))
             if (df->ws) (void)rocblas_set_workspace(h, nullptr, 0);
-        void* ps[] = {df->B, df->j2c, df->Y, df->X, df->part, df->D, df->rho, df->ws};
+        void* ps[] = {df->B, df->j2c, df->Y, df->kbuf, df->D, df->rho, df->ws};
         for (void* p : ps)
             if (p) (void)mjk_device_free(df->ctx, p);
     }

@@ -18,7 +18,7 @@ import numpy
 import pytest
 
 from pyscf_amd import df, gto, lib, workloads
-from pyscf_amd.scf import rhf
+from pyscf_amd.scf import _vhf, rhf
 
 pytestmark = pytest.mark.gpu
 H2O = 'O 0 0 0; H 0 -0.757 0.587; H 0 0.757 0.587'
@@ -214,3 +214,21 @@ def test_fit_factor_block_edges(n):
     ref = scipy.linalg.solve_triangular(L, raw, lower=True)
     fit = df.DF(mol, aux).build().cderi().reshape(n, -1)
     assert abs(fit - ref).max() <= 8 * n * 2.3e-16 * numpy.linalg.cond(L) * abs(ref).max()
+
+
+@pytest.mark.parametrize('size', [1, 4])
+def test_exchange_scratch_within_the_fit_workspace(size):
+    """A J/K call takes no device memory for its exchange products beyond the
+    half-transformed tensor: a budget of the fitted tensor, that and the call's
+    densities, J, K and fitting coefficients is enough."""
+    mol = gto.M(atom=workloads.water_cluster(size, shape=(4, 1, 1)), basis='cc-pvdz')
+    nao = mol.nao_nr()
+    dm = numpy.random.default_rng(size).standard_normal((nao, nao))
+    d = df.DF(mol, 'weigend', engine=_vhf.Engine()).build()
+    need = d.engine.hbm_used() + 8 * (d.get_naoaux() * (nao * nao + 1) + 3 * nao * nao)
+    ref = df.get_jk(d, dm, 0)
+    d2 = df.DF(mol, 'weigend', engine=_vhf.Engine(hbm_budget=need)).build()
+    out = df.get_jk(d2, dm, 0)
+    assert d2.engine.hbm_used() == need
+    for x, r in zip(out, ref):
+        assert abs(x - r).max() <= 1e-12 * abs(r).max()
