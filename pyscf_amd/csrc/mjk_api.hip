@@ -199,6 +199,7 @@ double flops_class(int a, int b, int c, int d, double nq, double nprimq, int nco
 struct mjk_ctx {
     int device = 0;
     int ncopy = 8;        // private J'/K' accumulator copies (MI355X has 8 XCDs)
+    bool jpairs = true;   // J' by shell pair where it fits
     // LDS bytes a row-kernel block may take; 0 = fallback kernels only.  gfx950
     // gives a workgroup up to 160 KB; 96 KB keeps room for a second block per CU
     // and let (dd|ss) on C30H62 cc-pVDZ use rows: 73.0 -> 68.9 ms per build
@@ -1521,6 +1522,13 @@ hipStream_t ctx_stream(mjk_ctx* ctx) { return ctx->stream; }
 int ctx_device(const mjk_ctx* ctx) { return ctx->device; }
 size_t ctx_budget(const mjk_ctx* ctx) { return ctx->budget; }
 std::recursive_mutex& ctx_mutex(mjk_ctx* ctx) { return ctx->mu; }
+Accumulators ctx_accumulators(const mjk_ctx* ctx) { return {ctx->ncopy, ctx->jpairs}; }
+void ctx_set_accumulators(mjk_ctx* ctx, const Accumulators& acc)
+{
+    std::lock_guard<std::recursive_mutex> lock(ctx->mu);
+    ctx->ncopy = acc.copies;
+    ctx->jpairs = acc.pairs;
+}
 std::shared_mutex& capture_mutex() { return g_capture; }
 void* ctx_blas(mjk_ctx* ctx) { return ctx->blas; }
 const double* ctx_rys(const mjk_ctx* ctx) { return ctx->rys; }
@@ -1800,7 +1808,7 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         if ((rc = ensure(ctx, &b->K, b->cap_k, ncopy * kcopy))) return rc;
         if (need_cond && (rc = ensure(ctx, &b->dmcond, b->cap_cond, b->cond_total))) return rc;
         // after all that the build must have: where it does not fit, every J' goes to the arena
-        if (jpcopy > 0 && ensure(ctx, &b->Jp, b->cap_jp, ncopy * jpcopy, false) == MJK_OK) Jpair = b->Jp;
+        if (ctx->jpairs && jpcopy > 0 && ensure(ctx, &b->Jp, b->cap_jp, ncopy * jpcopy, false) == MJK_OK) Jpair = b->Jp;
         Dj = b->Dj, Dk = b->Dk, Jacc = b->J, Kacc = b->K, dmcond = b->dmcond;
     } else {
         // each buffer starts on a 256-byte boundary; as many accumulator copies

@@ -31,6 +31,14 @@ void ctx_set_blas(mjk_ctx* ctx, void* handle, void (*destroy)(void*));
 void* ctx_rocblas(mjk_ctx* ctx);
 // Rys root table of the context (device)
 const double* ctx_rys(const mjk_ctx* ctx);
+// Private J'/K' accumulator copies of the context's builds, and whether they may
+// keep J' by shell pair too.
+struct Accumulators {
+    int copies = 1;
+    bool pairs = false;
+};
+Accumulators ctx_accumulators(const mjk_ctx* ctx);
+void ctx_set_accumulators(mjk_ctx* ctx, const Accumulators& acc);
 // density-fitted J and K of one density (device, nao x nao) with K from its
 // occupied orbitals X (device, column-major nao x nocc, D = X X^T)
 int df_get_jk_dev(mjk_df* df, const double* d_dm, const double* d_orbo_colmajor, int nocc, double* d_vj,

@@ -11,6 +11,8 @@
 //   free and the device bytes the contexts have tracked for their running
 //   requests (each request counted at least at its estimate until its
 //   buffers exist), plus the head's estimate, stay within the server's budget.
+//   Estimates are of the form that needs less memory; the fast form (J' by
+//   shell pair, all accumulator copies) runs where it keeps no one waiting.
 //   A request whose estimate alone exceeds the budget is refused at
 //   submission.
 // * Results stay in the server until mjk_result collects them.
@@ -32,12 +34,15 @@
 #include <vector>
 
 #include "mjk.h"
+#include "mjk_internal.h"
 
 namespace {
 
 constexpr int ATM_SLOTS = 6, BAS_SLOTS = 8;     // pyscf/gto/mole.py:80-101
 constexpr int CHARGE_OF = 0, PTR_COORD = 1;
 constexpr int ANG_OF = 1, NPRIM_OF = 2, NCTR_OF = 3;
+
+using mjk_internal::Accumulators;
 
 struct Req {
     long long ticket = 0;
@@ -47,7 +52,12 @@ struct Req {
     int natm = 0, nbas = 0, n_dm = 0, hermi = 1, with_j = 1, with_k = 1, nelectron = 0, max_cycle = 0;
     double direct_scf_tol = 0, fp32_tol = 0, conv_tol = 0;
     int nao = 0;
+    // bytes held at most and the accumulators that takes: as admitted (the
+    // smaller of the two forms below until then)
     size_t estimate = 0;
+    Accumulators acc;
+    size_t lean = 0, full = 0;
+    Accumulators acc_lean, acc_full;
     // results
     int state = MJK_REQ_QUEUED;
     std::vector<double> vj, vk, mo_energy;
@@ -71,6 +81,7 @@ struct Slot {
 struct mjk_server {
     int device = 0;
     size_t budget = 0;
+    Accumulators acc;                                 // as the slots' contexts take them by themselves
     std::vector<Slot> slots;
     std::mutex mu;
     std::condition_variable cv;
@@ -96,11 +107,16 @@ int nao_of(const std::vector<int>& bas, int nbas)
     return n;
 }
 
-// Upper estimate of the device bytes a request holds: primitive pairs (split
-// and merged representations), shell pairs, quartet task lists, the
-// Cartesian arenas (densities, the accumulator copies), J' by shell pair (at
-// most an arena per copy), dm_cond and, for an RHF, the SCF state.
-size_t estimate_bytes(const Req& r)
+// Upper estimates of the device bytes a request holds: primitive pairs (split
+// and merged representations), shell pairs, quartet task lists, the Cartesian
+// arenas (densities and accumulator copies; one density's worth even of the
+// part not asked for), J' by shell pair (an arena and at most four elements per
+// function, in every copy), dm_cond and, for an RHF, the SCF state.  In full:
+// the context's accumulator copies and J' by shell pair.  Lean: no J' by shell
+// pair and as many copies as 19 arenas per density hold (eight of a symmetric
+// J/K build, five of a general one), so that the fast form never keeps a
+// request from running.
+void estimate_bytes(Req& r, const Accumulators& acc)
 {
     double sp = 0, sp2 = 0;
     long long nsh = 0, ncart = 0;
@@ -117,11 +133,25 @@ size_t estimate_bytes(const Req& r)
     const double n = r.nao, nc = (double)ncart;
     const int ndm = std::max(r.n_dm, 1);
     double bytes = 48 * nprim_pairs + 160 * npairs + 16.0 * 55 * 16 * (npairs / 8 + 1) * 2;
-    bytes += 8.0 * (ndm * (3 + 3 * 8) * nc * nc + 3.0 * ndm * n * n + (double)nsh * nsh);
+    bytes += 8.0 * (3.0 * ndm * n * n + (double)nsh * nsh);
     // the SCF state: 15 n^2 matrices, two histories of 8, the solver workspace
     // (at least 4 n^2 doubles and 32 MiB), small vectors
     if (r.kind == MJK_REQ_RHF) bytes += 8.0 * (15 + 2 * 8 + 4 + 1) * n * n + (double)(32 << 20);
-    return (size_t)bytes + ((size_t)16 << 20);
+    const int n_j = r.with_j ? ndm : 0, n_k = r.with_k ? (r.hermi == 1 ? ndm : 2 * ndm) : 0;
+    const int slots = std::max(n_j, 1) + std::max(n_k, 1);
+    r.acc_full = acc;
+    r.acc_lean.pairs = false;
+    r.acc_lean.copies = std::max(1, std::min(acc.copies, 19 * ndm / slots - 1));
+    const double fixed = bytes + (double)((size_t)16 << 20);
+    r.lean = (size_t)(fixed + 8.0 * 19 * ndm * nc * nc);
+    r.full = (size_t)(fixed + 8.0 * ((1 + acc.copies) * (double)slots * nc * nc +
+                                     (acc.pairs ? acc.copies * (double)n_j * (nc * nc + 4 * nc) : 0.0)));
+    if (r.full <= r.lean) {
+        r.lean = r.full;
+        r.acc_lean = r.acc_full;
+    }
+    r.estimate = r.lean;
+    r.acc = r.acc_lean;
 }
 
 double nuclear_repulsion(const Req& r)
@@ -162,6 +192,7 @@ std::string ctx_error(mjk_ctx* ctx, int rc, const char* what)
 std::string execute(mjk_ctx* ctx, Req& r, size_t idle)
 {
     mjk_basis* b = nullptr;
+    mjk_internal::ctx_set_accumulators(ctx, r.acc);
     int rc = mjk_basis_upload(ctx, r.atm.data(), r.natm, r.bas.data(), r.nbas, r.env.data(), r.direct_scf_tol, &b);
     if (rc) return ctx_error(ctx, rc, "mjk_basis_upload");
     std::string err;
@@ -212,6 +243,18 @@ std::string execute(mjk_ctx* ctx, Req& r, size_t idle)
     return err;
 }
 
+// The full form of the request that starts now, if the idle slots could still
+// take a request each: as large as the largest waiting one, or as this one.
+void choose_form_locked(const mjk_server* s, Req& r)
+{
+    size_t idle = 0, next = r.lean;
+    for (const Slot& sl : s->slots) idle += !sl.running;
+    for (const auto& q : s->queue) next = std::max(next, q->lean);
+    const bool full = held_locked(s) + r.full + (idle - 1) * next <= s->budget;
+    r.estimate = full ? r.full : r.lean;
+    r.acc = full ? r.acc_full : r.acc_lean;
+}
+
 void worker(mjk_server* s, int k)
 {
     Slot& sl = s->slots[k];
@@ -226,6 +269,7 @@ void worker(mjk_server* s, int k)
             if (s->queue.empty()) return;
             r = s->queue.front();
             s->queue.pop_front();
+            choose_form_locked(s, *r);
             sl.running = r;
             r->state = MJK_REQ_RUNNING;
             r->slot = k;
@@ -298,6 +342,7 @@ int mjk_server_create(int device, int nslots, size_t hbm_budget, mjk_server** ou
         }
         s->slots[k].idle_bytes = mjk_ctx_hbm_used(s->slots[k].ctx);
     }
+    s->acc = mjk_internal::ctx_accumulators(s->slots[0].ctx);
     for (int k = 0; k < nslots; ++k) s->slots[k].th = std::thread(worker, s, k);
     *out = s;
     return MJK_OK;
@@ -338,7 +383,7 @@ int mjk_submit(mjk_server* s, const mjk_request* q, long long* ticket)
         r->max_cycle = q->max_cycle;
         r->conv_tol = q->conv_tol;
     }
-    r->estimate = estimate_bytes(*r);
+    estimate_bytes(*r, s->acc);
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->closing) return sfail(s, MJK_EINVAL, "server is closing");
     if (r->estimate > s->budget) {

@@ -94,3 +94,34 @@ def test_refusals():
     with pytest.raises(ValueError, match='even electron count'):
         srv.submit(Request('rhf', odd)).result(timeout=10)
     srv.close()
+
+
+@pytest.mark.parametrize('hermi', [0, 1])
+def test_estimate_holds_and_tight_budget_runs(hermi):
+    """Many densities, so that the arenas outweigh the estimate's reserves: the
+    tracked peak stays within the estimate, and a budget of 19 arenas per density
+    beside the fixed part (the full form takes 26 of a symmetric and 35 of a
+    general J/K build) still runs the request, with the same result."""
+    mol = gto.M(atom=workloads.water_cluster(4, shape=(4, 1, 1)), basis='cc-pvdz')
+    n, nd = mol.nao_nr(), 160
+    dms = numpy.random.default_rng(hermi).standard_normal((nd, n, n)) / n
+    if hermi:
+        dms = dms + dms.transpose(0, 2, 1)
+    j0, k0 = hf.get_jk(mol, dms, hermi)
+    arena = 8 * nd * (25 * 4) ** 2     # 25 Cartesian functions a molecule
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    lib.load_library().mjk_mem_info(0, ctypes.byref(free), ctypes.byref(total))
+    fraction, estimates = 0.8, []
+    for _ in range(2):
+        srv = JKServer(nslots=2, hbm_fraction=fraction)
+        req = Request('get_jk', mol, dms, hermi)
+        vj, vk = srv.submit(req).result(timeout=120)
+        srv.close()
+        print('hermi %d estimate %.1f MB peak %.1f MB' % (hermi, req.info.hbm_estimate / 2**20, req.info.hbm_peak / 2**20),
+              flush=True)
+        assert req.info.hbm_peak <= req.info.hbm_estimate <= srv.budget
+        for x, r in zip((vj, vk), (j0, k0)):
+            assert abs(x.reshape(r.shape) - r).max() <= 1e-12 * abs(r).max()
+        estimates.append(req.info.hbm_estimate)
+        fraction = (estimates[0] - (7 if hermi else 16) * arena) / total.value
+    assert estimates[1] < estimates[0]
