@@ -226,6 +226,16 @@ __host__ __device__ constexpr int jk_split(int la, int lb, int lc, int ld)
     return s.ka * s.kb * s.kc;
 }
 
+// Row classes with FP32 recurrences for small quartets (fp32_tol).  The heavier
+// ones stay in FP64 like the cooperative kernel that runs them where there are
+// fewer: FP32 took a mixed-precision build of a 598-AO def2-TZVP chain
+// (fp32_tol 1e-7) from 57.9 to 57.0 ms, and its error in K from 1.8e-13 to 6.1e-13.
+__host__ __device__ constexpr bool row_fp32(int la, int lb, int lc, int ld)
+{
+    const int nket = ncart(lc) * ncart(ld), nf = ncart(la) * ncart(lb) * nket;
+    return nf <= SLICE_NF || (nf <= 180 && nket <= 9);
+}
+
 struct QuartetCtx {
     int p, q, mol;
     bool alive, pvalid, qvalid;

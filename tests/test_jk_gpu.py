@@ -148,7 +148,9 @@ def test_row_kernel_b_rows_in_memory(oracle):
     (and below its full 13-20 rows), the (fp|..), (fd|..) and (ff|ss) classes
     run the row kernel that keeps the B rows of K' in memory; J and K equal
     the oracle's, for one density (one K' set) and for a non-symmetric one
-    (two)."""
+    (two).  (fp|ds) and (fd|ps), of two slices each, are asked for by tuning
+    entries: this molecule has too few of their quartets."""
+    from pyscf_amd import tune
     mol = gto.M(atom='O 0 0 0; H 0 -0.757 0.587; H 0 0.757 0.587; O 2.5 0.3 0.4', basis='def2-tzvp')
     nao = mol.nao_nr()
     bas = numpy.asarray(mol._bas)
@@ -156,19 +158,25 @@ def test_row_kernel_b_rows_in_memory(oracle):
     rng = numpy.random.default_rng(13)
     c = rng.standard_normal((nao, 8))
     eng = _vhf.get_engine()
+    saved = tune.read_table() if tune.load(eng) else []
     opt = _vhf.VHFOpt(mol, direct_scf_tol=1e-13)
+    sliced = [tune.class_key(opt.basis, cl[0]) for cl in opt.basis.classes(1, 1)
+              if cl[1] in ((3, 1, 2, 0), (3, 2, 1, 0))]
+    assert len(sliced) == 2
     try:
+        tune.set_table(eng, [dict(zip(tune.FIELDS[:9], k), kernel=1, rprim=0, scale=0.0) for k in sliced])
         for hermi, n_k, dm in ((1, 1, c @ c.T / 8), (0, 2, rng.standard_normal((nao, nao)))):
             lds = 8 * (n_k * 10 * ncart + 10 * 10)
             assert eng.lib.mjk_ctx_set_row_lds(eng.handle, lds) == 0
-            kinds = {cl[1]: cl[4] for cl in opt.basis.classes(1, hermi)}
-            assert kinds[(3, 1, 0, 0)] == 4 and kinds[(3, 1, 1, 0)] == 4 and kinds[(3, 3, 0, 0)] == 4, kinds
             vj, vk = hf.get_jk(mol, dm, hermi=hermi, vhfopt=opt)
+            kinds = {cl[1]: cl[4] for cl in opt.basis.classes(1, hermi)}
+            assert all(kinds[k] == 4 for k in ((3, 1, 0, 0), (3, 1, 1, 0), (3, 3, 0, 0), (3, 1, 2, 0), (3, 2, 1, 0))), kinds
             j0, k0 = oracle.get_jk(mol, dm, hermi=hermi)
             print('B rows in memory, hermi=%d: max|dJ|=%.2e max|dK|=%.2e' % (hermi, abs(vj - j0).max(),
                                                                          abs(vk - k0).max()), flush=True)
             assert abs(vj - j0).max() < TOL * max(1, abs(j0).max()) and abs(vk - k0).max() < TOL * max(1, abs(k0).max())
     finally:
+        tune.set_table(eng, saved)
         assert eng.lib.mjk_ctx_set_row_lds(eng.handle, 162816) == 0
 
 
@@ -351,13 +359,36 @@ def test_row_kernels_above_64k_lds(oracle):
     assert abs(j1[1] - jo).max() < 1e-9 and abs(k1[1] - ko).max() < 1e-9
 
 
+def sliced_classes_alone(eng, saved, b, build_jk):
+    """Classes of a basis whose row kernel is cut into slices, and what
+    build_jk(b) returns for each of them alone from the row kernel (1) and the
+    cooperative one (2)."""
+    from pyscf_amd import build, tune
+    sliced = [c for c in build.quartet_classes() if build.use_row(c) and build.jk_split(*c) > 1]
+    ks = [k for k, l, ctr, nb, kern in b.classes(2, 0) if tuple(l) in sliced and nb > 0]
+    assert len(ks) >= 15
+    out = {}
+    try:
+        for kernel in (1, 2):   # asked for by tuning entries: these molecules are small
+            tune.set_table(eng, [dict(zip(tune.FIELDS[:9], tune.class_key(b, k)), kernel=kernel, rprim=0, scale=0.0)
+                                 for k in ks])
+            for k in ks:
+                b.set_class_filter(k)
+                out[kernel, k] = build_jk(b)
+            assert [b.classes(2, 0)[k][4] for k in ks] == [kernel] * len(ks)
+    finally:
+        b.set_class_filter(-1)
+        tune.set_table(eng, saved)
+    return ks, out
+
+
 @pytest.mark.parametrize('omega', [None, 0.3])
 def test_sliced_row_classes_match_cooperative(omega):
     """Every quartet class whose row kernel is cut into slices (a, b or c blocks),
     alone, against its cooperative fallback.  The two add the same
     products in another order: a few thousand terms of size <= max|J'| at
     2^-53 each stay below 1e-12 of it."""
-    from pyscf_amd import build, tune
+    from pyscf_amd import tune
     mol = gto.M(atom='O 0 0 0; H 0 -0.757 0.587; H 0 0.757 0.587; O 2.5 0.3 0.4', basis='def2-tzvp')
     nao = mol.nao_nr()
     dms = numpy.random.default_rng(17).standard_normal((2, nao, nao))
@@ -365,26 +396,49 @@ def test_sliced_row_classes_match_cooperative(omega):
     saved = tune.read_table() if tune.load(eng) else []
     with mol.with_range_coulomb(omega):
         opt = _vhf.VHFOpt(mol, direct_scf_tol=1e-13)
-    b, out = opt.basis, {}
-    sliced = [c for c in build.quartet_classes() if build.use_row(c) and build.jk_split(*c) > 1]
-    ks = [k for k, l, ctr, nb, kern in b.classes(2, 0) if tuple(l) in sliced and nb > 0]
-    assert len(ks) >= 15
-    try:
-        for kernel in (1, 2):   # asked for by tuning entries: this molecule is small
-            tune.set_table(eng, [dict(zip(tune.FIELDS[:9], tune.class_key(b, k)), kernel=kernel, rprim=0, scale=0.0)
-                                 for k in ks])
-            for k in ks:
-                b.set_class_filter(k)
-                out[kernel, k] = b.get_jk(dms, 0, True, True, 1e-13)
-            assert [b.classes(2, 0)[k][4] for k in ks] == [kernel] * len(ks)
-    finally:
-        b.set_class_filter(-1)
-        tune.set_table(eng, saved)
+    ks, out = sliced_classes_alone(eng, saved, opt.basis, lambda b: b.get_jk(dms, 0, True, True, 1e-13))
     scale = [max(abs(out[1, k][i]).max() for k in ks) for i in (0, 1)]
     for k in ks:
         for i in (0, 1):
             d = abs(out[1, k][i] - out[2, k][i]).max()
             assert d < 1e-12 * max(1.0, scale[i]), (k, i, d)
+
+
+@pytest.mark.parametrize('fp32_tol', [0.0, 1e30])
+def test_sliced_row_classes_batched(fp32_tol):
+    """The same in a batch of which one molecule is inactive (task lists
+    compacted, blocks claiming tasks of every slice from its own counter), in
+    FP64 to 1e-12 as there, and with every quartet below fp32_tol.  Classes of
+    more than 180 components, or of more than 108 with more than nine in the ket,
+    have no FP32 recurrences in either kernel and stay at 1e-12.  In the others
+    all quartets of the row kernel run them: ten recurrence levels that may double
+    the rounding 6e-8 each give 6e-5 of the largest element, 1e-3 with room for
+    the class whose large terms cancel; a lost slice is of order one."""
+    from pyscf_amd import build, tune
+    atoms = ['O 0 0 0; H 0 -0.757 0.587; H 0 0.757 0.587; O 2.5 0.3 0.4', 'O 0 0 0; H 0 -0.757 0.587; H 0 0.757 0.587',
+             'C 0 0 0; O 0 0.3 2.3']
+    mols = [gto.M(atom=a, basis='def2-tzvp') for a in atoms]
+    eng = _vhf.get_engine()
+    saved = tune.read_table() if tune.load(eng) else []
+    b = eng.upload_batch(mols, 1e-13)
+    b.set_active([1, 0, 1])
+    rng = numpy.random.default_rng(19)
+    naos = [m.nao_nr() for m in mols]
+    dms = rng.standard_normal((2, sum(n * n for n in naos)))
+    ks, out = sliced_classes_alone(eng, saved, b, lambda b: b.get_jk(dms, 0, True, True, 1e-13, fp32_tol, stats=True)
+                                   + (b.last_stats['quartets'], b.last_stats['quartets_fp32']))
+    scale = [max(abs(out[2, k][i]).max() for k in ks) for i in (0, 1)]
+    idle = slice(naos[0] ** 2, naos[0] ** 2 + naos[1] ** 2)
+    l4 = {k: tuple(l) for k, l, *_ in b.classes(2, 0)}
+    for k in ks:
+        nf, nket = build.nfunc(l4[k]), build.ncart(l4[k][2]) * build.ncart(l4[k][3])
+        f32 = fp32_tol > 0 and nf <= 180 and nket <= 9
+        assert out[1, k][2] == out[2, k][2] > 0 and out[2, k][3] == 0, k
+        assert out[1, k][3] == (out[1, k][2] if f32 else 0), (l4[k], out[1, k][2:])
+        for i in (0, 1):
+            assert (out[1, k][i].reshape(2, -1)[:, idle] == 0).all()
+            d, own = abs(out[1, k][i] - out[2, k][i]).max(), abs(out[2, k][i]).max()
+            assert d < (1e-3 * own if f32 else 1e-12 * max(1.0, scale[i])), (l4[k], i, d, own)
 
 
 def test_builds_without_room_for_pair_accumulators():
