@@ -88,8 +88,9 @@ def use_row_m(c):
     shell above s, whose full rows pass a workgroup's 160 KB from about 1500
     Cartesian functions (13 to 20 rows) while their 10 A rows fit to 2000,
     cut into at most two slices.  Measured on MI355X (def2-TZVP chain, 1442
-    AOs, ms per launch, this kernel / the fallback): (fp|ps) 38.8 / 116.5
-    cooperative."""
+    AOs, ms per launch, this kernel / the fallback): (fp|ss) 10.8 / 40.2 tile,
+    (fp|ps) 19.5 / 104.5 cooperative, (fp|ds) 23.8 / 45.1, (fd|ss) 6.1 / 21.6
+    tile, (fd|ps) 24.1 / 43.1, (ff|ss) 3.6 / 12.2; the build 669 / 855."""
     return use_row(c) and c[0] == 3 and c[1] >= 1 and jk_split(*c) <= 2
 
 

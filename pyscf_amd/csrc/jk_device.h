@@ -203,8 +203,8 @@ __device__ __forceinline__ void count_work(unsigned long long* c, bool alive, in
 // registers (to 512) leave one wave per SIMD.  MI355X, def2-TZVP chain of 876
 // AOs, row kernel, ms in s slices: (fp|ps) 90 components 5: 15.0, 2: 7.5,
 // 1: 6.1; (dp|dp) 324 6: 6.6, 3: 4.9, 2: 15.1 (162 each spill); (fs|dp) 180
-// 5: 7.8, 2: 4.4; (fp|dp) 540 10: 9.9, 5: 7.3; (fp|pp) 270 5: 8.8, 2: 8.8,
-// 3 blocks of c: 7.8.
+// 5: 7.8, 2: 4.4; (fp|dp) 540 10: 9.9, 5: 7.3; (fp|pp) 270 5: 8.8, 2: 8.8, 3
+// blocks of c: 7.8, of b: 7.3.
 constexpr int SLICE_NF = 108;
 struct Slices {
     int ka, kb, kc;

@@ -17,8 +17,9 @@
 //     row i), then K = B^T Y over (P, l): K_ik = sum_Pl B_k[P,l] Y_i[P,l] =
 //     sum_P (B_P D B_P)_ik;
 //   * K of occupied orbitals X (D = X X^T): Y_i = B_i X, K = Y^T Y.
-// Both K products on the FP64 matrix cores (mjk_dfgemm.hip), also the
-// Cholesky factor; the fit's solve and eigenvectors on rocBLAS/rocSOLVER; everything on the context's stream, FP64 throughout.
+// Both K products and the Cholesky factor run on the FP64 matrix cores
+// (mjk_dfgemm.hip), the fit's solve and eigenvectors on rocBLAS/rocSOLVER;
+// everything on the context's stream, FP64 throughout.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>

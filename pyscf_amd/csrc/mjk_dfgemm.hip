@@ -370,8 +370,9 @@ __global__ __launch_bounds__(256) void k_chol_update(double* A, int n, int k0, i
 }  // namespace
 
 // Slices: waves in whole rounds of the card's 1024 SIMDs (a wave holds a SIMD
-// to itself), at least 256 inner elements each, the count with the fullest last
-// round within eight rounds; more slices only cost workspace traffic.
+// to itself).  Eight at least, one per XCD, however short; more while each keeps
+// 256 inner elements and all tiles fit eight rounds: the count with the fullest
+// last round, of about equals the smallest, as slices cost workspace traffic.
 TnPlan df_tn_plan(int n, long long kin, bool sym)
 {
     TnPlan p;

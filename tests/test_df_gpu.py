@@ -11,8 +11,9 @@ reference's golden values.
 * Golden values of pyscf/df/test/test_df_jk.py: lib.fp(vj), lib.fp(vk) of
   the seed-1 densities (9 places) and the DF-RHF energy (8 places).
 * K from occupied orbitals (the SCF path) equals K of their density.
-* The exchange GEMMs on even dimensions and in lower blocks (odd AO count,
-  forced blocks) against the oracle.
+* The matrix-core exchange products on odd and even AO counts against the
+  oracle, and at the edges of their tiles against numpy; the Cholesky factor at
+  the edges of its blocks, and the eigenvector fit where it fails.
 """
 import numpy
 import pytest
@@ -78,14 +79,11 @@ def test_fit_and_jk_vs_oracle(oracle, name):
         assert abs(vj - j0).max() <= TOL and abs(vk - k0).max() <= TOL
 
 
-@pytest.mark.parametrize('kblocks', ['0', '3'])
-def test_exchange_even_gemms_and_blocks(oracle, monkeypatch, kblocks):
-    """The exchange products run their GEMMs on an even number of AOs (an odd
-    last AO by matrix-vector products) and, with more than one block, as the
-    lower blocks of the symmetric product, mirrored: NH3 cc-pVDZ (29 AOs) and
+def test_exchange_odd_and_even_aos(oracle):
+    """The exchange products on the matrix cores, whose columns of an odd number of
+    AOs or fitting functions start at 8-byte addresses: NH3 cc-pVDZ (29 AOs) and
     H2O cc-pVDZ (24 AOs), general and occupied-orbital paths, against the
-    oracle's fit (kblocks 0 keeps one block at these sizes, 3 forces three)."""
-    monkeypatch.setenv('MJK_DF_KBLOCKS', kblocks)   # read when a DF object is built
+    oracle's fit."""
     nh3 = 'N 0 0 0.11; H 0 0.94 -0.26; H 0.81 -0.47 -0.26; H -0.81 -0.47 -0.26'
     for atom in (nh3, H2O):
         mol = gto.M(atom=atom, basis='cc-pvdz')
@@ -96,7 +94,7 @@ def test_exchange_even_gemms_and_blocks(oracle, monkeypatch, kblocks):
             dms = dens(nao, 11 + hermi, sym=sym)
             vj, vk = df.get_jk(d, dms, hermi)
             j0, k0 = oracle.df_get_jk(cd, dms, hermi)
-            print(nao, 'kblocks', kblocks, 'hermi=%d max|dJ|=%.2e max|dK|=%.2e'
+            print(nao, 'hermi=%d max|dJ|=%.2e max|dK|=%.2e'
                   % (hermi, abs(vj - j0).max(), abs(vk - k0).max()), flush=True)
             assert abs(vj - j0).max() <= TOL and abs(vk - k0).max() <= TOL
         rng = numpy.random.default_rng(3)
@@ -106,7 +104,7 @@ def test_exchange_even_gemms_and_blocks(oracle, monkeypatch, kblocks):
         dm = 2.0 * c[:, :5] @ c[:, :5].T
         vj, vk = df.get_jk(d, lib.tag_array(dm, mo_coeff=c, mo_occ=occ), 1)
         j0, k0 = oracle.df_get_jk(cd, dm[None], 1)
-        print(nao, 'kblocks', kblocks, 'orbitals max|dK|=%.2e' % abs(vk - k0[0]).max(), flush=True)
+        print(nao, 'orbitals max|dK|=%.2e' % abs(vk - k0[0]).max(), flush=True)
         assert abs(vj - j0[0]).max() <= TOL and abs(vk - k0[0]).max() <= TOL
 
 
@@ -232,3 +230,33 @@ def test_exchange_scratch_within_the_fit_workspace(size):
     assert d2.engine.hbm_used() == need
     for x, r in zip(out, ref):
         assert abs(x - r).max() <= 1e-12 * abs(r).max()
+
+
+def test_dependent_fitting_set_takes_the_eigenvector_fit():
+    """Forty nearly equal s functions on one centre: (P|Q) is singular to FP64
+    rounding (numpy's factorisation fails too), so the fit is over its
+    eigenvalues above lindep.  J and K against numpy's eigenvector fit of the
+    same integrals, which rounding of (P|Q) changes by up to
+    n eps w_max / w_min of the kept eigenvalues."""
+    mol = gto.M(atom=H2O, basis='cc-pvdz')
+    aux = {'O': [[0, (0.3 * 1.03 ** k, 1.0)] for k in range(40)], 'H': [[0, (0.8, 1.0)]]}
+    d = df.DF(mol, aux)
+    d.lindep = -1.0
+    raw = d.build().cderi()
+    n = raw.shape[0]
+    j2 = numpy.empty((n, n))
+    d.engine.check(d.engine.lib.mjk_df_fetch(d.engine.handle, d.handle, 0, j2.ctypes.data_as(lib.ctypes.c_void_p)),
+                   'mjk_df_fetch')
+    with pytest.raises(numpy.linalg.LinAlgError):
+        numpy.linalg.cholesky(j2)
+    w, v = numpy.linalg.eigh(j2)
+    keep = w > 1e-7
+    fit = df.DF(mol, aux).build()
+    assert fit.get_naoaux() == keep.sum() < n
+    b = numpy.einsum('pk,pij->kij', v[:, keep] / numpy.sqrt(w[keep]), raw)
+    dm = dens(mol.nao_nr(), 23)[0]
+    vj, vk = df.get_jk(fit, dm, 0)
+    j0 = numpy.einsum('pij,pkl,lk->ij', b, b, dm, optimize=True)
+    k0 = numpy.einsum('pij,jk,pkl->il', b, dm, b, optimize=True)
+    tol = n * 2.3e-16 * w[-1] / w[keep][0]
+    assert abs(vj - j0).max() <= tol * abs(j0).max() and abs(vk - k0).max() <= tol * abs(k0).max()
