@@ -562,6 +562,7 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
     }
     if (with_k) {
         const long long kin = (long long)naux * ncol;
+        const KLayout la = df_layout(nao, naux, ncol);
         const TnPlan plan = df_tn_plan(nao, std::max(kin, 1LL), d_orbo != nullptr);
         // scratch: padded orbitals (or density) of the half transform, slices of
         // the product.  The fit's workspace (32 MiB, or a copy of B for the
@@ -588,11 +589,12 @@ int get_jk_dev(mjk_df* df, const double* d_dms, int n_dm, const double* d_orbo, 
             const double* M = d_orbo ? d_orbo + (size_t)k * nao * nocc : d_dms + (size_t)k * nn;
             const bool cm = d_orbo && orbo_colmajor;
             if (df_pad_x(M, cm ? 1 : ncol, cm ? nao : 1, nao, ncol, X, st) ||
-                df_y(df->B, X, nao, naux, ncol, df->Y, st))
+                df_y(df->B, X, nao, naux, ncol, la, df->Y, st))
                 return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: half-transform launch failed");
             // K = Y^T Y over (P, o), symmetric; or K (row-major) = B^T Y over
-            // (P, l): column-major C(k, i) = K[i][k]
-            if (df_tn(plan, d_orbo ? df->Y : df->B, df->Y, nao, kin, d_orbo != nullptr, part, K, st))
+            // (P, l): column-major C(k, i) = K[i][k] (B read by column too, as
+            // it is symmetric in k and l)
+            if (df_tn(plan, d_orbo ? df->Y : df->B, df->Y, nao, kin, la, d_orbo != nullptr, part, K, st))
                 return ctx_fail(ctx, MJK_EDEVICE, "mjk_df: exchange product launch failed");
         }
     }

@@ -13,10 +13,11 @@
 //            reading B and the matrix cores.
 //
 // Measured on MI355X.  C18H38 cc-pVDZ (442 AOs, 73 orbitals, 2126 fitting
-// functions): K product 25.0 -> 0.58 ms (53 TFLOP/s; rocBLAS DGEMM ran it on
-// 12 tiles of 128 x 192), half transform 1.94 -> 1.56 ms (39 TFLOP/s, 43 with
-// the padding of 73 columns to 80); the J/K call 28.8 -> 3.1 ms.  A
-// nine-heavy-atom chain, def2-SVP, general density: K product 26.9 -> 0.33 ms.
+// functions), library products -> these kernels: K product 25.0 -> 0.65 ms
+// (rocBLAS DGEMM ran it on 12 tiles of 128 x 192), half transform 1.94 -> 1.39 ms
+// (44 TFLOP/s, 48 with the padding of 73 columns to 80).  C30H62 (730 AOs, 3526
+// functions): 121 orbitals 5.7 -> 4.3 and 8.7 -> 8.1 ms, general density 51.3 ->
+// 46.5 and 42.2 -> 43.6 ms.
 #include "df_gemm.h"
 
 #include <algorithm>
@@ -88,22 +89,24 @@ __device__ __forceinline__ void tn_tile(int t, int nt, bool sym, int& ti, int& t
 
 // One wave per (tile, slice); the tiles of one slice run on one XCD (blocks go
 // to the XCDs in turn), whose L2 then serves the slice's rows to all of them.
+// Inner element k of row i at (k / np) os + i is + k % np (KLayout).
 __global__ void __launch_bounds__(256, 1) k_df_tn(const double* __restrict__ A, const double* __restrict__ B, int n,
-                                                 long long kin, TnPlan pl, int sym, double* __restrict__ part)
+                                                 long long kin, KLayout la, TnPlan pl, int sym,
+                                                 double* __restrict__ part)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, q = lane >> 4;
     const int idx = (blockIdx.x >> 3) * 4 + wave;
     const int s = (idx / pl.ntile) * 8 + (blockIdx.x & 7), t = idx % pl.ntile;
     if (s >= pl.nsplit) return;
-    const long long k0 = s * pl.kc, k1 = min(k0 + pl.kc, kin);
+    const long long end = min((s + 1) * pl.kc, kin);
     int ti, tj;
     tn_tile(t, pl.nt, sym != 0, ti, tj);
-    const double *pa[4], *pb[4];
+    long long ra[4], rb[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) {   // rows past the last are computed on the last row and dropped
-        pa[g] = A + min(ti * 64 + 16 * g + m, n - 1) * kin + 4 * q;
-        pb[g] = B + min(tj * 64 + 16 * g + m, n - 1) * kin + 4 * q;
+        ra[g] = min(ti * 64 + 16 * g + m, n - 1) * la.is + 4 * q;
+        rb[g] = min(tj * 64 + 16 * g + m, n - 1) * la.is + 4 * q;
     }
     v4d acc[4][4];
 #pragma unroll
@@ -111,33 +114,43 @@ __global__ void __launch_bounds__(256, 1) k_df_tn(const double* __restrict__ A, 
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = v4d{0, 0, 0, 0};
     double a0[4][4], b0[4][4], a1[4][4], b1[4][4];
-    long long k = k0;
-    const long long kf = k0 + ((k1 - k0) & ~15LL);   // whole sixteens (k1 < k0: none)
-    if (k + 16 <= kf) {
-        tn_load(pa, k, a0);
-        tn_load(pb, k, b0);
-        for (; k + 48 <= kf; k += 32) {   // the next sixteen in flight behind 64 MFMAs
-            tn_load(pa, k + 16, a1);
-            tn_load(pb, k + 16, b1);
-            tn_mul(a0, b0, acc);
-            tn_load(pa, k + 32, a0);
-            tn_load(pb, k + 32, b0);
-            tn_mul(a1, b1, acc);
+    for (long long at = s * pl.kc; at < end;) {   // the contiguous runs of the slice
+        const long long o = at / la.np;
+        long long k = at - o * la.np;
+        const long long k1 = min(la.np, k + end - at), kf = k + ((k1 - k) & ~15LL);   // whole sixteens
+        at += k1 - k;
+        const double *pa[4], *pb[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            pa[g] = A + o * la.os + ra[g];
+            pb[g] = B + o * la.os + rb[g];
         }
-        tn_mul(a0, b0, acc);
-        k += 16;
         if (k + 16 <= kf) {
             tn_load(pa, k, a0);
             tn_load(pb, k, b0);
+            for (; k + 48 <= kf; k += 32) {   // the next sixteen in flight behind 64 MFMAs
+                tn_load(pa, k + 16, a1);
+                tn_load(pb, k + 16, b1);
+                tn_mul(a0, b0, acc);
+                tn_load(pa, k + 32, a0);
+                tn_load(pb, k + 32, b0);
+                tn_mul(a1, b1, acc);
+            }
             tn_mul(a0, b0, acc);
             k += 16;
+            if (k + 16 <= kf) {
+                tn_load(pa, k, a0);
+                tn_load(pb, k, b0);
+                tn_mul(a0, b0, acc);
+                k += 16;
+            }
         }
-    }
-    if (k < k1) {
-        const int rest = (int)min(4LL, max(0LL, k1 - k - 4 * q));
-        tn_load_tail(pa, k, rest, a0);
-        tn_load_tail(pb, k, rest, b0);
-        tn_mul(a0, b0, acc);
+        if (k < k1) {
+            const int rest = (int)min(4LL, max(0LL, k1 - k - 4 * q));
+            tn_load_tail(pa, k, rest, a0);
+            tn_load_tail(pb, k, rest, b0);
+            tn_mul(a0, b0, acc);
+        }
     }
     double* out = part + ((long long)s * pl.ntile + t) * 4096 + lane;
 #pragma unroll
@@ -175,9 +188,19 @@ __global__ void __launch_bounds__(256) k_df_tn_sum(const double* __restrict__ pa
 // element l + q (512 contiguous bytes per element over the 16 m), which are
 // row m of the wave's four 16-row groups.  The panels of one (i, row tile) are
 // neighbouring waves, so B_i comes from memory once.
+//   Every load is unconditional, at a clamped address where there is nothing to
+// load (the last functions once more, stored again with the same value; the
+// last inner element, times a zero row of X): a load under a condition makes
+// the compiler wait for all loads at the join, those of the next step with
+// them, and nothing is in flight behind the products.  Eight inner elements a
+// step: two waves per SIMD to five groups.  MI355X, ms, conditional loads of
+// sixteen elements / these: 442 AOs and 73 orbitals 1.67 / 1.39, 730 and 121
+// 10.9 / 8.1, general density of 730 85.9 / 43.6 (63 TFLOP/s; spilled registers
+// of six groups had their part in it; the library's DGEMM 42.2).
+constexpr int Y_U = 2;   // groups of four inner elements a step
 template <int NSUB>
 __global__ void __launch_bounds__(256, 1) k_df_y(const double* __restrict__ B, const double* __restrict__ Xp, int nao,
-                                             int naux, int ncol, int ldx, int npan, double* __restrict__ Y)
+                                             int naux, int ncol, int ldx, int npan, KLayout la, double* __restrict__ Y)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, q = lane >> 4;
@@ -187,82 +210,90 @@ __global__ void __launch_bounds__(256, 1) k_df_y(const double* __restrict__ B, c
     const int tm = (int)((item / npan) % ntm);
     const long long i = item / ((long long)npan * ntm);
     if (i >= nao) return;
-    const int p0 = tm * 64 + 4 * m;
-    const bool whole = tm * 64 + 64 <= naux;   // wave-uniform
-    const double* b = B + i * nao * naux + p0 + (long long)q * naux;
-    const double* x = Xp + (long long)q * ldx + pan * 16 * NSUB + m;
+    const double* b = B + i * nao * naux + min(tm * 64 + 4 * m, naux - 4);
+    const double* x = Xp + pan * 16 * NSUB + m;
     v4d acc[4][NSUB];
 #pragma unroll
     for (int g = 0; g < 4; ++g)
 #pragma unroll
         for (int j = 0; j < NSUB; ++j) acc[g][j] = v4d{0, 0, 0, 0};
-    constexpr int U = 4;   // groups of four inner elements per step
-    const int lw = whole ? nao & ~15 : 0;
-    auto load = [&](int l, double (&ab)[U][4], double (&xb)[U][NSUB]) {
+    auto load = [&](int l, double (&ab)[Y_U][4], double (&xb)[Y_U][NSUB]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int le = l + 4 * u;
-            if (l < lw) {
-                const d2u lo = *(const d2u*)(b + (long long)le * naux), hi = *(const d2u*)(b + (long long)le * naux + 2);
-                ab[u][0] = lo.x;
-                ab[u][1] = lo.y;
-                ab[u][2] = hi.x;
-                ab[u][3] = hi.y;
-            } else {
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    ab[u][g] = le + q < nao && p0 + g < naux ? b[(long long)le * naux + g] : 0.0;
-            }
+        for (int u = 0; u < Y_U; ++u) {
+            const int le = l + 4 * u + q;
+            const double* bl = b + (long long)min(le, nao - 1) * naux;
+            const d2u lo = *(const d2u*)bl, hi = *(const d2u*)(bl + 2);
+            ab[u][0] = lo.x;
+            ab[u][1] = lo.y;
+            ab[u][2] = hi.x;
+            ab[u][3] = hi.y;
 #pragma unroll
             for (int j = 0; j < NSUB; ++j) xb[u][j] = x[(long long)le * ldx + 16 * j];   // rows padded to sixteens
         }
     };
-    auto mul = [&](const double (&ab)[U][4], const double (&xb)[U][NSUB]) {
+    auto mul = [&](const double (&ab)[Y_U][4], const double (&xb)[Y_U][NSUB]) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < Y_U; ++u)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
 #pragma unroll
                 for (int j = 0; j < NSUB; ++j) acc[g][j] = mfma(ab[u][g], xb[u][j], acc[g][j]);
     };
-    double a0[U][4], x0[U][NSUB], a1[U][4], x1[U][NSUB];
+    double a0[Y_U][4], x0[Y_U][NSUB], a1[Y_U][4], x1[Y_U][NSUB];
+    constexpr int STEP = 4 * Y_U;
+    const int ns = (nao + STEP - 1) / STEP;
     load(0, a0, x0);
-    for (int l = 0; l < nao; l += 32) {   // the next sixteen elements in flight behind the products
-        if (l + 16 < nao) load(l + 16, a1, x1);
+    for (int s = 0; s < ns; s += 2) {   // the next step in flight behind the products (the last one loaded again)
+        load(STEP * min(s + 1, ns - 1), a1, x1);
         mul(a0, x0);
-        if (l + 16 >= nao) break;
-        if (l + 32 < nao) load(l + 32, a0, x0);
-        mul(a1, x1);
+        load(STEP * min(s + 2, ns - 1), a0, x0);
+        if (s + 1 < ns) mul(a1, x1);
     }
     // lane (m, q): orbital m of sub-panel j, fitting functions 4 (4 v + q) .. + 3
-    double* y = Y + i * naux * ncol;
+    double* y = Y + i * la.is;
 #pragma unroll
     for (int j = 0; j < NSUB; ++j) {
         const int o = (pan * NSUB + j) * 16 + m;
         if (o >= ncol) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int p = tm * 64 + 4 * (4 * v + q);
-            double* d = y + (long long)o * naux + p;
-            if (whole) {
-                *(d2u*)d = d2u{acc[0][j][v], acc[1][j][v]};
-                *(d2u*)(d + 2) = d2u{acc[2][j][v], acc[3][j][v]};
-            } else {
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    if (p + g < naux) d[g] = acc[g][j][v];
-            }
+            double* d = y + o * la.yo + min(tm * 64 + 4 * (4 * v + q), naux - 4);
+            *(d2u*)d = d2u{acc[0][j][v], acc[1][j][v]};
+            *(d2u*)(d + 2) = d2u{acc[2][j][v], acc[3][j][v]};
         }
     }
 }
 
-// Panels of the orbitals: at most six 16-column groups per wave (192
-// accumulator registers), as few panels as that allows, equally wide.
+// The same for fewer than four fitting functions, an element per thread.
+__global__ void __launch_bounds__(256) k_df_y_few(const double* __restrict__ B, const double* __restrict__ Xp, int nao,
+                                                 int naux, int ncol, int ldx, KLayout la, double* __restrict__ Y)
+{
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (long long)nao * ncol * naux) return;
+    const int p = (int)(e % naux), o = (int)(e / naux % ncol);
+    const long long i = e / ((long long)naux * ncol);
+    double v = 0.0;
+    for (int l = 0; l < nao; ++l) v = fma(B[(i * nao + l) * naux + p], Xp[(long long)l * ldx + o], v);
+    Y[i * la.is + o * la.yo + p] = v;
+}
+
+// Panels of the orbitals, at most five 16-column groups per wave (two waves per
+// SIMD): the fewest groups with the padding, a panel counted as 0.4 more for
+// its reads of B.  MI355X, 730 AOs, ms: 730 columns in 12 panels of 4 groups
+// 43.6, in 8 of 6 49.2; 442 AOs: 73 columns in one of 5 1.38, in two of 3 1.60.
 void y_panels(int ncol, int& nsub, int& npan)
 {
     const int n = (ncol + 15) / 16;
-    npan = (n + 5) / 6;
-    nsub = (n + npan - 1) / npan;
+    double best = 0;
+    nsub = 0;
+    for (int k = 5; k >= 1; --k) {
+        const int np = (n + k - 1) / k;
+        if (nsub == 0 || np * (k + 0.4) < best) {
+            best = np * (k + 0.4);
+            nsub = k;
+            npan = np;
+        }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_df_pad_x(const double* __restrict__ src, long long sl, long long so, int nao,
@@ -373,6 +404,7 @@ __global__ __launch_bounds__(256) void k_chol_update(double* A, int n, int k0, i
 // to itself).  Eight at least, one per XCD, however short; more while each keeps
 // 256 inner elements and all tiles fit eight rounds: the count with the fullest
 // last round, of about equals the smallest, as slices cost workspace traffic.
+constexpr long long TN_SLICE = 16384;
 TnPlan df_tn_plan(int n, long long kin, bool sym)
 {
     TnPlan p;
@@ -389,16 +421,19 @@ TnPlan df_tn_plan(int n, long long kin, bool sym)
             p.nsplit = s;
         }
     }
+    // tiles of a slice drift apart in a long one and no longer find each other's
+    // rows in L2: 730 AOs, general density, 56 slices of 46 000 49.9 ms, 128 46.8
+    p.nsplit *= (int)std::max(1LL, (kin / p.nsplit + TN_SLICE - 1) / TN_SLICE);
     p.kc = ((kin + p.nsplit - 1) / p.nsplit + 15) / 16 * 16;
     p.ws = (size_t)p.nsplit * p.ntile * 4096;
     return p;
 }
 
-int df_tn(const TnPlan& pl, const double* A, const double* B, int n, long long kin, bool sym, double* part, double* C,
-          hipStream_t st)
+int df_tn(const TnPlan& pl, const double* A, const double* B, int n, long long kin, const KLayout& la, bool sym,
+          double* part, double* C, hipStream_t st)
 {
     const int per_xcd = pl.nsplit / 8 * pl.ntile;
-    k_df_tn<<<(unsigned)((per_xcd + 3) / 4 * 8), 256, 0, st>>>(A, B, n, kin, pl, sym, part);
+    k_df_tn<<<(unsigned)((per_xcd + 3) / 4 * 8), 256, 0, st>>>(A, B, n, kin, la, pl, sym, part);
     k_df_tn_sum<<<(unsigned)(pl.ntile * 16), 256, 0, st>>>(part, pl, n, sym, C);
     return (int)hipGetLastError();
 }
@@ -419,20 +454,36 @@ int df_pad_x(const double* src, long long sl, long long so, int nao, int ncol, d
     return (int)hipGetLastError();
 }
 
-int df_y(const double* B, const double* Xp, int nao, int naux, int ncol, double* Y, hipStream_t st)
+// By row up to 2 MB a row, above by column: the 128 rows that a tile's wave reads
+// side by side then lie within a few pages instead of one page each.  MI355X,
+// K product, ms, by row / by column: 442 AOs, kin 156 000 0.68 / 0.69, 472 000
+// 1.90 / 1.72; 730 AOs, 212 000 2.30 / 2.36, 427 000 4.59 / 4.26, 1.3 million
+// 15.7 / 11.8, general density (2.6 million) 68.4 / 49.9.
+KLayout df_layout(int nao, int naux, int ncol)
+{
+    const long long kin = (long long)naux * ncol, col = (long long)nao * naux;
+    if (kin * (long long)sizeof(double) < (2LL << 20)) return {kin, kin, 0, naux};
+    return {naux, naux, col, col};
+}
+
+int df_y(const double* B, const double* Xp, int nao, int naux, int ncol, const KLayout& la, double* Y, hipStream_t st)
 {
     int nsub, npan;
     y_panels(ncol, nsub, npan);
     const int ldx = nsub * npan * 16;
+    if (naux < 4) {
+        const long long n = (long long)nao * ncol * naux;
+        k_df_y_few<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, la, Y);
+        return (int)hipGetLastError();
+    }
     const long long items = (long long)nao * ((naux + 63) / 64) * npan;
     const unsigned nb = (unsigned)((items + 3) / 4);
     switch (nsub) {
-    case 1: k_df_y<1><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
-    case 2: k_df_y<2><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
-    case 3: k_df_y<3><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
-    case 4: k_df_y<4><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
-    case 5: k_df_y<5><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
-    default: k_df_y<6><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, Y); break;
+    case 1: k_df_y<1><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, la, Y); break;
+    case 2: k_df_y<2><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, la, Y); break;
+    case 3: k_df_y<3><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, la, Y); break;
+    case 4: k_df_y<4><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, la, Y); break;
+    default: k_df_y<5><<<nb, 256, 0, st>>>(B, Xp, nao, naux, ncol, ldx, npan, la, Y); break;
     }
     return (int)hipGetLastError();
 }

@@ -260,3 +260,46 @@ def test_dependent_fitting_set_takes_the_eigenvector_fit():
     k0 = numpy.einsum('pij,jk,pkl->il', b, dm, b, optimize=True)
     tol = n * 2.3e-16 * w[-1] / w[keep][0]
     assert abs(vj - j0).max() <= tol * abs(j0).max() and abs(vk - k0).max() <= tol * abs(k0).max()
+
+
+def test_exchange_layout_by_column():
+    """The half-transformed tensor is laid out by column from 2 MB a row on:
+    orbital counts on both sides of that line (923 fitting functions, so 284 of
+    them) and a general density (312 columns) against numpy on the fitted tensor,
+    1e-12 of the largest element as for the small ones."""
+    mol = gto.M(atom=workloads.water_cluster(13, shape=(4, 4, 1)), basis='cc-pvdz')
+    d = df.DF(mol, 'weigend').build()
+    b = d.cderi()
+    naux, nao = b.shape[:2]
+    assert (naux, nao) == (923, 312)
+    rng = numpy.random.default_rng(13)
+    for nocc in (284, 285, 0):
+        if nocc:
+            c = rng.standard_normal((nao, nocc)) / 10
+            vk = df.get_jk(d, lib.tag_array(c @ c.T, mo_coeff=c, mo_occ=numpy.ones(nocc)), 1, with_j=False)[1]
+            y = (b.reshape(-1, nao) @ c).reshape(naux, nao, nocc)
+            k0 = sum(yp @ yp.T for yp in y)
+            assert (vk == vk.T).all()
+        else:
+            dm = rng.standard_normal((nao, nao)) / 10
+            vk = df.get_jk(d, dm, 0, with_j=False)[1]
+            y = (b.reshape(-1, nao) @ dm).reshape(naux, nao, nao)
+            k0 = sum(yp @ bp for yp, bp in zip(y, b))
+        assert abs(vk - k0).max() <= 1e-12 * abs(k0).max(), nocc
+
+
+@pytest.mark.parametrize('n', [1, 2, 3, 4, 5])
+def test_exchange_few_fitting_functions(n):
+    """Fewer fitting functions than a lane loads at once, and just as many."""
+    mol = gto.M(atom=[('H', (0, 0, 1.1 * i)) for i in range(n)], basis='cc-pvdz', spin=n % 2)
+    d = df.DF(mol, {'H': [[0, (0.8, 1.0)]]}).build()
+    b = d.cderi()
+    nao = b.shape[1]
+    rng = numpy.random.default_rng(n)
+    c = rng.standard_normal((nao, 3))
+    vk = df.get_jk(d, lib.tag_array(c @ c.T, mo_coeff=c, mo_occ=numpy.ones(3)), 1)[1]
+    y = numpy.einsum('pij,jo->pio', b, c)
+    assert b.shape[0] == n and abs(vk - numpy.einsum('pio,pjo->ij', y, y)).max() <= 1e-12 * abs(vk).max()
+    dm = rng.standard_normal((nao, nao))
+    vk = df.get_jk(d, dm, 0)[1]
+    assert abs(vk - numpy.einsum('pij,jk,pkl->il', b, dm, b)).max() <= 1e-12 * abs(vk).max()
