@@ -133,6 +133,19 @@ struct JKArgs {
     int ntask;
 };
 
+// Arrays that one launch clears (a launch of a replayed graph costs a small
+// molecule's build about as much as its smaller classes, 5 us on MI355X).
+struct ZeroArgs {
+    double* p[5];
+    long long n[5];
+    int count = 0;
+    void add(void* dst, long long doubles)
+    {
+        p[count] = (double*)dst;
+        n[count++] = doubles;
+    }
+};
+
 // One pair group's part of the J' accumulators by shell pair.
 struct JGroup {
     long long e0;           // first element

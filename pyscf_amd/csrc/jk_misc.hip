@@ -149,11 +149,14 @@ __global__ __launch_bounds__(256) void k_sph2cart(const XformArgs x, const doubl
     }
 }
 
-// Sum of an accumulator's private copies into the first one, before the output
-// transform, which then reads one copy (it reads each element up to 36 times).
-// Bandwidth-bound.
-__global__ __launch_bounds__(256) void k_sum_copies(double* __restrict__ acc, long long n, int ncopy, long long copy)
+// Sum of the accumulators' private copies (y = 0: J', 1: K') into the first
+// one, before the output transform, which then reads one copy (it reads each
+// element up to 36 times).  Bandwidth-bound.
+__global__ __launch_bounds__(256) void k_sum_copies(double* __restrict__ J, long long nj, long long jcopy,
+                                                    double* __restrict__ K, long long nk, long long kcopy, int ncopy)
 {
+    double* acc = blockIdx.y ? K : J;
+    const long long n = blockIdx.y ? nk : nj, copy = blockIdx.y ? kcopy : jcopy;
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
         double v = 0.0;
         for (int c = 0; c < ncopy; ++c) v += acc[c * copy + e];
@@ -161,11 +164,13 @@ __global__ __launch_bounds__(256) void k_sum_copies(double* __restrict__ acc, lo
     }
 }
 
-int launch_sum_copies(double* acc, long long n, int ncopy, long long copy, hipStream_t st)
+int launch_sum_copies(double* J, long long nj, long long jcopy, double* K, long long nk, long long kcopy, int ncopy,
+                      hipStream_t st)
 {
+    const long long n = std::max(nj, nk);
     if (n <= 0 || ncopy < 2) return 0;
     const long long nb = std::min<long long>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_sum_copies, dim3((unsigned)nb), dim3(256), 0, st, acc, n, ncopy, copy);
+    hipLaunchKernelGGL(k_sum_copies, dim3((unsigned)nb, 2), dim3(256), 0, st, J, nj, jcopy, K, nk, kcopy, ncopy);
     return (int)hipGetLastError();
 }
 
@@ -284,8 +289,10 @@ __global__ __launch_bounds__(256) void k_copy(const double* __restrict__ src, do
 
 // Zero fill (a kernel rather than a memset node, so that a captured graph
 // replays it like any other kernel).
-__global__ __launch_bounds__(256) void k_zero(double* __restrict__ dst, long long n)
+__global__ __launch_bounds__(256) void k_zero(const ZeroArgs a)
 {
+    double* __restrict__ dst = a.p[blockIdx.y];
+    const long long n = a.n[blockIdx.y];
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         dst[i] = 0.0;
 }
@@ -320,11 +327,13 @@ int launch_compact_rows(const int4* rt, int nrt, const int* pmol, const int* act
     return (int)hipGetLastError();
 }
 
-int launch_zero(double* dst, long long n, hipStream_t st)
+int launch_zero(const ZeroArgs& a, hipStream_t st)
 {
+    long long n = 0;
+    for (int i = 0; i < a.count; ++i) n = std::max(n, a.n[i]);
     if (n <= 0) return 0;
     const long long nb = std::min<long long>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)nb), dim3(256), 0, st, dst, n);
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)nb, (unsigned)a.count), dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
 

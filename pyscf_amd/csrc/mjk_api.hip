@@ -60,7 +60,8 @@ int launch_sph2cart(const XformArgs& x, int maxld, const double* Dsph, long long
 int launch_cart2sph(const XformArgs& x, int maxnao, const double* Jc, const double* Kc, long long cslot,
                     int n_dm, int hermi, int with_j, int with_k, double* vj, double* vk, long long sslot,
                     hipStream_t st);
-int launch_sum_copies(double* acc, long long n, int ncopy, long long copy, hipStream_t st);
+int launch_sum_copies(double* J, long long nj, long long jcopy, double* K, long long nk, long long kcopy, int ncopy,
+                      hipStream_t st);
 int launch_jscatter(const ScatterArgs& a, hipStream_t st);
 int launch_compact_rows(const int4* rt, int nrt, const int* pmol, const int* active, int* list, int* count,
                         hipStream_t st);
@@ -68,7 +69,7 @@ int launch_dmcond(const DmCondArgs& x, const double* Dsph, long long sslot, int 
                   hipStream_t st);
 int lmax_kernels();
 int launch_copy(const double* src, double* dst, long long n, hipStream_t st);
-int launch_zero(double* dst, long long n, hipStream_t st);
+int launch_zero(const ZeroArgs& a, hipStream_t st);
 }  // namespace mjk
 
 using namespace mjk;
@@ -1841,12 +1842,18 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     // accumulators are cleared by a kernel, not a memset node.
     auto enqueue = [&](bool capture) -> int {
     if (!capture) HIPCHK(ctx, hipEventRecord(ctx->ev[0], st));
-    if (n_j && (launch_zero(Jacc, ncopy * jcopy, st) || (Jpair && launch_zero(Jpair, ncopy * jpcopy, st))))
-        return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
-    if (n_k && launch_zero(Kacc, ncopy * kcopy, st)) return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
-    // (the 64-bit counters are cleared as doubles: both are all-zero bits)
-    if (tally && launch_zero(reinterpret_cast<double*>(b->counters), 4 * NQCLASS_MAX, st))
-        return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
+    // persistent row launches: the blocks claim tasks from a counter; a batched
+    // basis first compacts the tasks of its active molecules into a list
+    const bool persist = ctx->persist == 2 || (ctx->persist == 1 && b->nmol > 1);
+    const bool compact = persist && b->nmol > 1;
+    ZeroArgs clear;
+    if (n_j) clear.add(Jacc, ncopy * jcopy);
+    if (Jpair) clear.add(Jpair, ncopy * jpcopy);
+    if (n_k) clear.add(Kacc, ncopy * kcopy);
+    // (the integer counters are cleared as doubles: both are all-zero bits)
+    if (tally) clear.add(b->counters, 4 * NQCLASS_MAX);
+    if (persist) clear.add(b->d_tctl, ROW_TCTL / 2 * NQCLASS_MAX);
+    if (launch_zero(clear, st)) return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
     if (need_cond && launch_dmcond(dmcond_args(b), d_dms, b->slot_s, n_dm, dmcond, st))
         return fail(ctx, MJK_EDEVICE, "dm_cond launch failed");
     if (launch_sph2cart(xform(b), b->maxld, d_dms, b->slot_s, n_dm, hermi, with_j, with_k, Dj, Dk,
@@ -1882,12 +1889,6 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
     a.tcount = nullptr;
     a.thead = nullptr;
     a.ntask = 0;
-    // persistent row launches: the blocks claim tasks from a counter; a batched
-    // basis first compacts the tasks of its active molecules into a list
-    const bool persist = ctx->persist == 2 || (ctx->persist == 1 && b->nmol > 1);
-    const bool compact = persist && b->nmol > 1;
-    if (persist && launch_zero(reinterpret_cast<double*>(b->d_tctl), ROW_TCTL / 2 * NQCLASS_MAX, st))
-        return fail(ctx, MJK_EDEVICE, "zero fill launch failed");
     // classes, heaviest first, each on the least loaded of the streams (they all
     // add into the same J'/K' with atomics, so their order does not matter)
     const int nst = ctx->nstreams;
@@ -1997,8 +1998,7 @@ static int get_jk_impl(mjk_ctx* ctx, mjk_basis* b, const double* d_dms, int n_dm
         HIPCHK(ctx, hipStreamWaitEvent(st, ctx->ev_join[i - 1], 0));
     }
     if (!capture) HIPCHK(ctx, hipEventRecord(ctx->ev[2], st));
-    if (launch_sum_copies(Kacc, n_k * b->slot_c, ncopy, kcopy, st) ||
-        launch_sum_copies(Jacc, n_j * b->slot_c, ncopy, jcopy, st))
+    if (launch_sum_copies(Jacc, n_j * b->slot_c, jcopy, Kacc, n_k * b->slot_c, kcopy, ncopy, st))
         return fail(ctx, MJK_EDEVICE, "accumulator sum launch failed");
     if (Jpair) {
         ScatterArgs sa;
