@@ -614,17 +614,27 @@ int build_tiles(mjk_basis* b, double cutoff)
             if ((rc = upload(ctx, btm, &qc.bt_mol))) return rc;
             if ((rc = upload(ctx, off, &qc.bt_off))) return rc;
         }
-        // A sliced row kernel (one quartet per lane, every slice a pass over the
-        // class) needs quartets to fill its lanes; below about 30 000 per slice
-        // the cooperative kernel (one quartet per block) is done before a pass's
-        // latency is over.  MI355X, ms, row / cooperative: (dd|ds) in 2 slices
-        // 28 k quartets 0.23 / 0.22, 130 k 0.35 / 0.64; (dd|pp) in 3 32 k 0.44 /
-        // 0.30, 74 k 0.67 / 0.57, 288 k 0.74 / 1.40; (dd|dp) in 6 65 k 0.70 /
-        // 0.53, 136 k 0.75 / 0.89; (fd|dp) in 10 61 k 1.27 / 0.82, 1.1 M 5.8 /
-        // 10.9.  A tuning entry may ask for either.
-        const bool merged = qc.ca * qc.cb * qc.cc * qc.cd > 1;
+        // A row kernel of more than 81 components (one quartet per lane, each of
+        // its slices a pass over the class) needs quartets to fill its lanes; below
+        // about 30 000 per slice the cooperative kernel (one quartet per block) is
+        // done before a pass's latency is over.  MI355X, ms, row / cooperative:
+        // (dd|ds) in 2 slices 28 k quartets 0.23 / 0.22, 130 k 0.35 / 0.64; (dd|pp)
+        // in 3 32 k 0.44 / 0.30, 74 k 0.67 / 0.57, 288 k 0.74 / 1.40; (dd|dp) in 6
+        // 65 k 0.70 / 0.53, 136 k 0.75 / 0.89; (fd|dp) in 10 61 k 1.27 / 0.82, 1.1 M
+        // 5.8 / 10.9.  Beside the other streams' kernels a wave that fills a SIMD's
+        // registers also waits for one to be empty, and whole builds turn later than
+        // the class alone: C14H30 cc-pVDZ with (dp|dp) (3 slices, 95 k quartets, alone
+        // 0.45 / 0.60) 10.35 / 9.32, C18H38 14.7 / 14.8, so 60 000 from three slices
+        // on.  In one slice ((dp|ds), (dd|ps)) 15 000: (H2O)4 cc-pVDZ 1.64 / 1.42,
+        // C6H14 3.52 / 3.30, C8H18 5.38 / 5.02, C9H20 5.79 / 5.89 with 30 000.
+        // Classes with f shells turn with the class alone (their cooperative kernels
+        // are the slower ones) and in one slice never.  A tuning entry may ask for
+        // either.
+        const bool merged = qc.ca * qc.cb * qc.cc * qc.cd > 1, f = qc.la > 2;
         const int slices = merged ? 1 : row_kernel_slices(qc.la, qc.lb, qc.lc, qc.ld);
-        const bool few = slices > 1 && qc.kernel_pref != 1 && est_q < 3.0e4 * slices;
+        const bool wide = !merged && ncart(qc.la) * ncart(qc.lb) * ncart(qc.lc) * ncart(qc.ld) > 81;
+        const bool few = wide && slices > (f ? 1 : 0) && qc.kernel_pref != 1 &&
+                         est_q < (f || slices == 2 ? 3.0e4 : slices == 1 ? 1.5e4 : 6.0e4) * slices;
         // Row-kernel tasks: the same Schwarz prefixes per bra pair, cut into
         // chunks of about equal primitive-quartet count (the kets' primitive
         // counts differ up to a hundredfold).
