@@ -675,8 +675,8 @@ def bench_df(args):
         'paths_agree': {'max_dJ': float(abs(vj - vj2).max()), 'max_dK': float(abs(vk - vk2).max())},
         'roofline': {'bound': 'mfma', 'achieved': flops_mo / t_mo * 1e-12, 'peak': FP64_PEAK * 1e-12,
                      'unit': 'TFLOP/s', 'frac': flops_mo / t_mo / FP64_PEAK, 'traffic': None,
-                     'note': 'whole build (J two passes over the tensor; K a strided-batched rocBLAS FP64 GEMM and '
-                             'the symmetric product as lower blocks), algorithmic FLOPs (the symmetric product '
+                     'note': 'whole build (J two passes over the tensor; K the half transform and the lower tiles '
+                             'of the symmetric product), algorithmic FLOPs (the symmetric product '
                              'counted once per unique element) over wall time per synchronised build'},
         'cpu_baseline': None,
     }
